@@ -192,17 +192,17 @@ void decode_swiglu(const uint16_t* x, const uint8_t* codes, const float* scales,
 void linear_candidates_impl(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t S, int64_t M,
                             int64_t N, int64_t K, int64_t offset, void* ws, double* out, hipStream_t stream);
 
-void gemm_bf16_impl(const uint16_t* x, const uint16_t* w, uint16_t* y, int64_t ldy, int64_t M,
+// y = x * w^T (+ bias) for BF16 weights; y rounded before the bias is added.
+void gemm_bf16_impl(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int64_t M,
                     int64_t N, int64_t K, hipStream_t stream) {
     if (M <= 8) {
         const bool wide = K % 16 == 0 && aligned16(x) && aligned16(w);
         check_hip(fp8lin::launch_gemv(x, w, false, nullptr, 1, y, ldy, (int)M, (int)N, (int)K, wide,
                                       stream),
                   "bf16 gemv launch");
+        if (bias) check_hip(fp8lin::launch_bias(y, ldy, bias, M, N, stream), "bias launch");
     } else {
-        check_hip(fp8lin::launch_gemm(x, w, nullptr, 1, y, ldy, (int)M, (int)N, (int)K, false,
-                                      stream),
-                  "bf16 gemm launch");
+        check_hip(fp8lin::launch_gemm_bf16(x, w, bias, y, ldy, (int)M, (int)N, (int)K, stream), "bf16 gemm launch");
     }
 }
 
@@ -318,8 +318,9 @@ void validate_engine(const fp8lin_linear_options& o, const fp8lin_weight& w, con
     if (w.scales) check_scales(w.scales, w.scale_cols, w.K);
 }
 
+// bias_added: set where the branch's kernel added w.bias itself.
 int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const uint16_t* x,
-                  int64_t rows, uint16_t* y, int64_t ldy, void* ws, size_t ws_bytes,
+                  int64_t rows, uint16_t* y, int64_t ldy, void* ws, size_t ws_bytes, bool& bias_added,
                   hipStream_t stream) {
     const auto* codes = static_cast<const uint8_t*>(w.data);
     // src/engine.cpp:206-213
@@ -339,7 +340,8 @@ int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const 
     }
     // :220-221
     if (w.cached_bf16 && rows > 1) {
-        gemm_bf16_impl(x, w.cached_bf16, y, ldy, rows, w.N, w.K, stream);
+        gemm_bf16_impl(x, w.cached_bf16, w.bias, y, ldy, rows, w.N, w.K, stream);
+        bias_added = true;
         return FP8LIN_PATH_CACHED_BF16;
     }
     // :222-224
@@ -368,12 +370,13 @@ int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const 
             check_hip(fp8lin::launch_dequant(codes + begin * w.K, s, w.scale_cols, slab, w.K, count,
                                              w.K, stream),
                       "dequant launch");
-            gemm_bf16_impl(x, slab, y + begin, ldy, rows, count, w.K, stream);
+            gemm_bf16_impl(x, slab, nullptr, y + begin, ldy, rows, count, w.K, stream);
         }
         return FP8LIN_PATH_DEQUANT_GEMM;
     }
     // :234-237
-    gemm_bf16_impl(x, static_cast<const uint16_t*>(w.data), y, ldy, rows, w.N, w.K, stream);
+    gemm_bf16_impl(x, static_cast<const uint16_t*>(w.data), w.bias, y, ldy, rows, w.N, w.K, stream);
+    bias_added = true;
     return FP8LIN_PATH_BF16;
 }
 
@@ -382,8 +385,9 @@ int engine_impl(const fp8lin_linear_options& o, const fp8lin_weight& w, const ui
                 int64_t rows, uint16_t* y, int64_t ldy, void* ws, size_t ws_bytes,
                 hipStream_t stream) {
     validate_engine(o, w, x, rows, y, ldy);
-    const int path = engine_branch(o, w, x, rows, y, ldy, ws, ws_bytes, stream);
-    if (w.bias) check_hip(fp8lin::launch_bias(y, ldy, w.bias, rows, w.N, stream), "bias launch");
+    bool bias_added = false;
+    const int path = engine_branch(o, w, x, rows, y, ldy, ws, ws_bytes, bias_added, stream);
+    if (w.bias && !bias_added) check_hip(fp8lin::launch_bias(y, ldy, w.bias, rows, w.N, stream), "bias launch");
     return path;
 }
 
@@ -640,7 +644,7 @@ int fp8lin_gemm_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, int64_t 
         check_dims(M, N, K);
         require(ldy >= N, FP8LIN_ERR_SHAPE, "BF16 GEMM: ldy < N");
         ensure_device();
-        gemm_bf16_impl(x, w, y, ldy, M, N, K, as_stream(stream));
+        gemm_bf16_impl(x, w, nullptr, y, ldy, M, N, K, as_stream(stream));
     });
 }
 

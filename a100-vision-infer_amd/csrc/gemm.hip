@@ -255,4 +255,13 @@ hipError_t launch_gemm(const uint16_t* x, const void* w, const float* scales, in
                   : run<false, false>(x, w, nullptr, 1, y, ldy, M, N, K, stream);
 }
 
+hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
+                            int N, int K, hipStream_t stream) {
+    if (!skinny(M, N, false) && tile_supported(x, w, false, 1, M, N, K))
+        return launch_tile(tile_plan(false, 1, M, N, K, false), false, x, w, nullptr, 1, bias, y, ldy, M, N, K, false,
+                           nullptr, stream);
+    const hipError_t e = launch_gemm(x, w, nullptr, 1, y, ldy, M, N, K, false, stream);
+    return e != hipSuccess || !bias ? e : launch_bias(y, ldy, bias, M, N, stream);
+}
+
 }  // namespace fp8lin

@@ -1,0 +1,152 @@
+// Dispatch of the one-tile-per-workgroup GEMM (gemm_tile.hpp): which tile, how
+// wide its column blocks are and into how many K ranges it is cut.
+#include <algorithm>
+
+#include "gemm_tile.hpp"
+#include "internal.hpp"
+
+namespace fp8lin {
+namespace {
+
+using gemm_tile::Cfg;
+using gemm_tile::Grid;
+
+typedef hipError_t (*LaunchFn)(const uint16_t*, const void*, const float*, int, const uint16_t*, uint16_t*, int64_t,
+                               int, int, int, const Grid&, float*, hipStream_t);
+
+// One tile configuration and what a round of it costs: tau is the measured
+// time in us of 128 K with the whole chip running it (one workgroup per CU;
+// `slots` 2: two per CU, tau for both, tau1 where one per CU is enough).
+struct Tile {
+    int bm, bn, slots;
+    float tau, tau1;
+    LaunchFn plain, swiglu;
+    int (*lds)(int, int, int);
+};
+
+template <class C, bool FP8>
+constexpr Tile tile(int slots, float tau, float tau1) {
+    return {C::BM, C::BN, slots, tau, tau1, gemm_tile::launch<C, false>, FP8 ? gemm_tile::launch<C, FP8> : nullptr, C::lds_bytes};
+}
+
+// BF16 weights, M x N x K in us (torch's mm, hipBLASLt, beside it): 1036 x 3456
+// x 1152 13.4 (24.5), 1036 x 4304 x 1152 19.7 (21.1), 1036 x 1152 x 4304 28
+// (31), 40 x 7168 x 5120 19.9 (22.3), 300 x 5120 x 5120 30.5 (35.8), 4096 x
+// 8192 x 8192 456 (355: the library's large tile is the better one).  The
+// 256x256-only kernel this replaced took 47, 46, 571 (K % 64 != 0), 159.
+// Small tiles split a step's K over the waves of the workgroup, so that a
+// wave's tile stays deep enough for its LDS reads; FP8 tiles keep WM = 1 up
+// to 128 rows, where every code is dequantized once.
+const Tile kBf16[] = {
+    tile<Cfg<false, 32, 32, 1, 1, 4, 128, 6, false>, false>(1, 0.25f, 0.25f),
+    tile<Cfg<false, 64, 32, 1, 1, 4, 128, 3, false>, false>(1, 0.39f, 0.39f),
+    tile<Cfg<false, 64, 64, 1, 2, 4, 128, 3, false>, false>(1, 0.49f, 0.49f),
+    tile<Cfg<false, 128, 64, 2, 1, 4, 128, 3, false>, false>(1, 0.68f, 0.68f),
+    tile<Cfg<false, 128, 128, 2, 2, 2, 64, 4, true>, false>(1, 0.98f, 0.98f),
+    tile<Cfg<false, 128, 128, 2, 2, 1, 64, 2, false>, false>(2, 1.80f, 1.15f),
+    tile<Cfg<false, 256, 256, 2, 4, 1, 64, 2, false>, false>(1, 2.95f, 2.95f),
+};
+const Tile kFp8[] = {
+    tile<Cfg<true, 32, 32, 1, 1, 4, 128, 8, false>, true>(1, 0.34f, 0.34f),
+    tile<Cfg<true, 64, 32, 1, 1, 4, 128, 4, false>, true>(1, 0.38f, 0.38f),
+    tile<Cfg<true, 64, 64, 1, 2, 4, 128, 4, false>, true>(1, 0.51f, 0.51f),
+    tile<Cfg<true, 96, 64, 1, 2, 4, 128, 4, false>, true>(1, 0.60f, 0.60f),
+    tile<Cfg<true, 128, 64, 1, 2, 4, 128, 3, false>, true>(1, 0.70f, 0.70f),
+    tile<Cfg<true, 64, 128, 1, 2, 4, 128, 4, false>, true>(1, 0.76f, 0.76f),
+    tile<Cfg<true, 96, 192, 1, 6, 2, 64, 5, true>, true>(1, 1.37f, 1.37f),
+    tile<Cfg<true, 128, 128, 1, 4, 2, 64, 5, true>, true>(1, 1.27f, 1.27f),
+    tile<Cfg<true, 256, 128, 2, 4, 1, 64, 3, true>, true>(1, 2.00f, 2.00f),
+    tile<Cfg<true, 256, 256, 2, 4, 1, 64, 2, false>, true>(1, 3.20f, 3.20f),
+};
+constexpr int kMaxTileSplits = 8;
+
+int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
+
+// Microseconds of tile t over M x N x K in `splits` K ranges: launch, first
+// loads and last stores; the rounds of workgroups, each over its K range; and
+// for a split the partials written and read back and the second launch.
+float estimate(const Tile& t, int M, int N, int K, int splits, int cus) {
+    const int64_t units = (int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
+    const int steps = ceil_div(ceil_div(K, 128), splits);
+    const bool single = units <= cus;
+    const float rounds = single ? 1.0f : (float)ceil_div(units, (int64_t)cus * t.slots);
+    const float us = 4.0f + rounds * (float)steps * (single ? t.tau1 : t.tau);
+    return splits == 1 ? us : us + 4.0f + 8.0e-6f * (float)splits * (float)M * (float)N / 6.0f;
+}
+
+const Tile& tile_of(bool fp8, int i) { return fp8 ? kFp8[i] : kBf16[i]; }
+
+Grid grid_of(const Tile& t, int M, int N, int64_t ldy, const uint16_t* y, const uint16_t* bias, int splits, bool swiglu,
+             int cus) {
+    Grid g;
+    g.mtiles = ceil_div(M, t.bm);
+    g.nblocks = ceil_div(N, t.bn);
+    g.splits = splits;
+    g.group_m = 8;
+    g.ldp = ceil_div(N, 8) * 8 + 8;
+    g.wide = (ldy % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 ? 1 : 0) |
+             (reinterpret_cast<uintptr_t>(bias) % 16 == 0 ? 2 : 0);
+    // One round: spread the columns evenly over the CUs.
+    g.per = t.bn;
+    const int fit = cus / (g.mtiles * splits);
+    if (fit >= g.nblocks) {
+        g.per = std::min(t.bn, ceil_div(ceil_div(N, fit), 16) * 16);
+        g.nblocks = ceil_div(N, g.per);
+    }
+    if (swiglu && splits == 1) g.per /= 2;
+    return g;
+}
+
+}  // namespace
+
+bool tile_supported(const uint16_t* x, const void* w, bool fp8, int S, int64_t M, int64_t N, int64_t K) {
+    const int64_t lim = (int64_t)1 << 31;
+    return M > 0 && K % (fp8 ? 16 : 8) == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(w) % 16 == 0 && N * K * (fp8 ? 1 : 2) < lim && 256 * K * 2 < lim &&
+           N + 16 < lim / 8 && M < lim / 8 && (!fp8 || S == 1 || S == (K + 127) / 128);
+}
+
+// The plan with the smallest estimate.  It depends on M, N, K, S and whether
+// a split may be taken, not on the epilogue, so that the SwiGLU form sums as
+// the plain one.
+TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split) {
+    const int cus = compute_units(), count = fp8 ? (int)(sizeof(kFp8) / sizeof(Tile)) : (int)(sizeof(kBf16) / sizeof(Tile));
+    TilePlan best{-1, 1, 0.0f};
+    for (int i = 0; i < count; ++i) {
+        const Tile& t = tile_of(fp8, i);
+        const int64_t tiles = (int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn);
+        const int most = may_split ? std::min(kMaxTileSplits, ceil_div(K, 128)) : 1;
+        for (int s = 1; s <= most && (s == 1 || tiles * s <= cus); ++s) {
+            if (t.lds(S, K, s) > gemm_tile::kLds) continue;
+            const float us = estimate(t, M, N, K, s, cus);
+            if (best.cfg < 0 || us < best.us) best = {i, s, us};
+        }
+    }
+    return best;
+}
+
+size_t tile_plan_bytes(const TilePlan& p, int M, int N) {
+    return p.splits == 1 ? 0 : (size_t)p.splits * M * (ceil_div(N, 8) * 8 + 8) * sizeof(float);
+}
+
+hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,
+                       const uint16_t* bias, uint16_t* y, int64_t ldy, int M, int N, int K, bool swiglu, void* ws,
+                       hipStream_t stream) {
+    const Tile& t = tile_of(fp8, p.cfg);
+    const Grid g = grid_of(t, M, N, ldy, y, bias, p.splits, swiglu, compute_units());
+    float* part = static_cast<float*>(ws);
+    if (p.splits == 1) return (swiglu ? t.swiglu : t.plain)(x, w, scales, S, bias, y, ldy, M, N, K, g, nullptr, stream);
+    const hipError_t e = t.plain(x, w, scales, S, nullptr, y, ldy, M, N, K, g, part, stream);
+    if (e != hipSuccess) return e;
+    const int64_t threads = (int64_t)M * ceil_div(swiglu ? N >> 1 : N, 8);
+    const dim3 grid((unsigned)((threads + 255) / 256));
+    if (swiglu)
+        hipLaunchKernelGGL(gemm_tile::split_reduce_kernel<true>, grid, dim3(256), 0, stream, part, g.splits, g.ldp, bias, y,
+                           ldy, M, N, g.wide);
+    else
+        hipLaunchKernelGGL(gemm_tile::split_reduce_kernel<false>, grid, dim3(256), 0, stream, part, g.splits, g.ldp, bias, y,
+                           ldy, M, N, g.wide);
+    return hipGetLastError();
+}
+
+}  // namespace fp8lin

@@ -1,0 +1,510 @@
+// GEMM over one output tile per workgroup: y[M,N] = x[M,K] * W^T (+ bias) on
+// the BF16 matrix cores, W as BF16 or as E4M3FN codes with FP32 scales (per
+// row or per 128-K block), any K whose rows start on 16 bytes.
+//
+// Orientation: the weights are the MFMA's A operand and the activations its B
+// operand, so a lane's 16 accumulator values are outputs of one activation
+// row.  Weight row n of a 32-row fragment sits at fragment row i(n) with
+// n = 16 h + 4 q + t for i = 8 q + 4 h + t, which makes the 16 values
+// consecutive columns: two 16-byte stores per fragment.
+//
+// A workgroup of WM x WN x WK waves computes a BM x BN tile; a wave owns
+// (BM / WM) x (BN / WN) of it as 32x32 accumulators, over every WK-th 32-K
+// slice of a step (WK > 1: the WK partial tiles are added in LDS in wave
+// order at the end).  Splitting K over waves instead of splitting the tile
+// keeps the wave's tile, and with it the LDS reads per MFMA, while a second
+// wave per SIMD hides the first one's LDS and barrier waits; with WM == 1 it
+// also dequantizes every FP8 code once per workgroup.
+//
+// Data movement: BK of K per step through a ring of ST stages, filled by
+// direct-to-LDS DMA ST - 1 steps ahead, one wait and one barrier per step.
+// The 16-byte chunks of a row are XOR-swizzled so that the 16 rows of a
+// fragment read fall in distinct LDS banks.  K is cut in 16-byte chunks:
+// chunks at or past K, rows past M and weight rows past N read zeros, and
+// every step issues the same number of DMAs, so the waits are fixed numbers.
+#pragma once
+#include "device.hpp"
+#include "gemm_fp8.hpp"
+
+namespace fp8lin {
+namespace gemm_tile {
+
+using gemm_fp8::dma16;
+using gemm_fp8::i32x4;
+using gemm_fp8::make_desc;
+
+constexpr int kLds = 160 * 1024;
+
+// 128-K scale blocks that a K range of kt steps may touch.
+template <class C>
+__host__ __device__ inline int scale_blocks(int S, int kt) {
+    if (S == 1) return 1;
+    const int b = kt * C::BK / 128 + (C::BK < 128 ? 2 : 1);
+    return b < S ? b : S;
+}
+
+// PIPE: the next slice's fragments are read (and dequantized) into a second
+// register set while the current ones are multiplied; stage t + 1 must then
+// have landed before step t, one stage less in flight.  It gains 5-8% where a
+// step has enough MFMAs to cover the reads (128 x 128 tiles at ST >= 4) and
+// loses a few percent on small tiles, and on tiles that only fit two stages.
+template <bool FP8_, int BM_, int BN_, int WM_, int WN_, int WK_, int BK_, int ST_, bool PIPE_>
+struct Cfg {
+    static constexpr bool PIPE = PIPE_;
+    static constexpr bool FP8 = FP8_;
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, WK = WK_, BK = BK_, ST = ST_;
+    static constexpr int WAVES = WM * WN * WK, THREADS = 64 * WAVES;
+    static constexpr int MT = BM / WM / 32, NT = BN / WN / 32;  // 32x32 accumulators per wave
+    static constexpr int XROW = 2 * BK, WROW = FP8 ? BK : 2 * BK;  // LDS row bytes of a stage
+    static constexpr int X_STAGE = BM * XROW, W_STAGE = BN * WROW, STAGE = X_STAGE + W_STAGE;
+    static constexpr int XD = X_STAGE / 1024 / WAVES, WD = W_STAGE / 1024 / WAVES;  // DMAs per wave and step
+    static constexpr int ND = XD + WD;
+    static constexpr int RING = ST * STAGE;
+    static constexpr int SLICES = BK / 32;  // 32-K slices (two MFMAs deep) of a step
+    static_assert(BK == 32 || BK == 64 || BK == 128, "stages of whole 32-K slices");
+    static_assert(ST >= (PIPE ? 3 : 2), "a stage in flight beside the ones read");
+    static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && SLICES % WK == 0, "wave tile");
+    static_assert(X_STAGE % (1024 * WAVES) == 0 && W_STAGE % (1024 * WAVES) == 0, "equal DMA shares");
+    static_assert(WK == 1 || BM * BN * 4 <= RING, "a partial tile fits the ring");
+    static_assert(RING <= kLds, "LDS");
+    // Ring and, for FP8, the rows' scales of the longest K range, padded to an
+    // odd stride so that 32 rows at one block fall in distinct banks.
+    static int lds_bytes(int S, int K, int splits) {
+        const int ksteps = (K + BK - 1) / BK, kt = (ksteps + splits - 1) / splits;
+        return RING + (FP8 ? BN * (scale_blocks<Cfg>(S, kt) | 1) * 4 : 0);
+    }
+};
+
+// o = bf16(y + bias) of eight rounded outputs from column c on, as the separate
+// bias kernel adds it; wide: eight bias values in one load where all are below lim.
+__device__ __forceinline__ void add_bias8(uint32_t* o, const uint16_t* __restrict__ bias, int c, int lim, bool wide) {
+    uint32_t v[4];
+    if (wide && c + 8 <= lim) {
+        const u32x4 q = load_u32x4(bias + c);
+        v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            v[r] = (c + 2 * r < lim ? (uint32_t)bias[c + 2 * r] : 0u) |
+                   (c + 2 * r + 1 < lim ? (uint32_t)bias[c + 2 * r + 1] << 16 : 0u);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        o[r] = pack_bf16x2(f32x2{bf16_bits_to_f32(o[r] & 0xffffu) + bf16_bits_to_f32(v[r] & 0xffffu),
+                                 bf16_bits_to_f32(o[r] >> 16) + bf16_bits_to_f32(v[r] >> 16)});
+}
+
+// Position of chunk ch of row r in a row of CH chunks.
+template <int CH>
+__device__ __forceinline__ int swz(int r, int ch) {
+    if constexpr (CH == 16) return ch ^ (r & 15);
+    if constexpr (CH == 8) return ch ^ gemm_fp8::ga(r);
+    if constexpr (CH == 4) return ch ^ gemm_fp8::gb(r);
+    return ch ^ ((r >> 2) & 1);
+}
+
+// Column of fragment row i (0..31) in its 32-column block (see the header).
+__device__ __forceinline__ int frag_col(int i) { return 16 * ((i >> 2) & 1) + 4 * (i >> 3) + (i & 3); }
+
+// Waits until at most N of the wave's DMAs are in flight and its LDS reads are
+// done, then for the workgroup.
+template <int N>
+__device__ __forceinline__ void wait_vm_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+}
+
+// 16-byte chunk at LDS byte address a.
+__device__ __forceinline__ u32x4 lds16(uint32_t a) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)a);
+}
+
+// Weight row of tile row b (fragment order) of the column block that starts at
+// row (SWIGLU: output) n0 and holds `per` of them, or -1.  SWIGLU: the 32 rows
+// of a fragment are 16 outputs; lane half h's 16 values are the gates of
+// outputs 8 h + [0, 8), then their ups.
+template <bool SWIGLU>
+__device__ __forceinline__ int64_t weight_row(int n0, int per, int b, int N) {
+    const int c = frag_col(b & 31);
+    if constexpr (SWIGLU) {
+        const int D = N >> 1, r = (b >> 5) * 16 + 8 * (c >> 4) + (c & 7), o = n0 + r;
+        return r < per && o < D ? ((c & 8) ? (int64_t)D + o : (int64_t)o) : -1;
+    } else {
+        const int r = (b & ~31) + c;
+        return r < per && n0 + r < N ? (int64_t)n0 + r : -1;
+    }
+}
+
+// Work of one launch: column blocks of `per` outputs (SWIGLU: output pairs),
+// at most a tile's width, and `splits` K ranges of whole steps each, whose
+// FP32 sums go to part[split][M][ldp] for split_reduce_kernel.  per below the
+// tile's width lets the blocks match the CU count; the rows past it cost no
+// memory traffic.
+struct Grid {
+    int mtiles, nblocks, per, splits;
+    int group_m;  // tile rows walked together (x and W rows shared in an XCD's L2)
+    int ldp;      // row stride of the partials
+    int wide;     // 1: y rows hold 16-byte aligned 8-column groups; 2: so does bias
+};
+
+// Requirements (checked by the launcher): x, w 16-byte aligned; K % 8 == 0
+// (BF16) or K % 16 == 0 (FP8); BM * K * 2 and N * K * (FP8 ? 1 : 2) below
+// 2^31; S == 1 or ceil(K / 128); per % 8 == 0 and per <= BN (SWIGLU: BN / 2).
+// With SWIGLU, N counts weight rows and y is [M, N/2].
+template <class C, bool SWIGLU>
+__global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
+                                                               const float* __restrict__ scales, int S,
+                                                               const uint16_t* __restrict__ bias,
+                                                               uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K,
+                                                               Grid gr, float* __restrict__ part) {
+    extern __shared__ __align__(16) uint8_t smem[];
+    constexpr int CHX = C::BK / 8, CHW = C::FP8 ? C::BK / 16 : C::BK / 8;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = lane >> 5, l32 = lane & 31;
+    const int wk = wave / (C::WM * C::WN), wm = wave / C::WN % C::WM, wn = wave % C::WN;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
+
+    // Unit of this workgroup: each XCD (workgroup % 8) takes a contiguous run
+    // of the units (split, tile), a split's tiles walked group_m tile rows at
+    // a time, so that the tiles an XCD runs together share x and W rows in
+    // its L2.
+    const int tiles = gr.mtiles * gr.nblocks, units = tiles * gr.splits;
+    const int per_xcd = (units + 7) / 8;
+    const int u = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    if ((int)(blockIdx.x / 8) >= per_xcd || u >= units) return;
+    const int split = u / tiles, L = u - split * tiles;
+    const int per_group = gr.group_m * gr.nblocks, g = L / per_group;
+    const int gsize = min(gr.group_m, gr.mtiles - g * gr.group_m), rem = L - g * per_group;
+    const int m0 = (g * gr.group_m + rem % gsize) * C::BM, n0 = rem / gsize * gr.per;
+    const int ksteps = (K + C::BK - 1) / C::BK;
+    const int t0 = (int)((int64_t)ksteps * split / gr.splits), KT = (int)((int64_t)ksteps * (split + 1) / gr.splits) - t0;
+
+    const int rows = min(C::BM, M - m0);
+    const i32x4 dx = make_desc(x + (int64_t)m0 * K, (uint32_t)((int64_t)rows * K * 2));
+    const i32x4 dw = make_desc(w, (uint32_t)((int64_t)N * K * (C::FP8 ? 1 : 2)));
+
+    // DMA d of this wave fills 1 KiB of a stage: lane -> byte 16 * lane of it.
+    uint32_t xoff[C::XD], woff[C::WD];
+    int xk[C::XD], wk0[C::WD];  // first K of the lane's chunk within a step
+#pragma unroll
+    for (int d = 0; d < C::XD; ++d) {
+        const int q = (wave * C::XD + d) * 64 + lane, r = q / CHX, ch = swz<CHX>(r, q % CHX);
+        xk[d] = 8 * ch;
+        xoff[d] = r < rows ? (uint32_t)(r * K * 2 + ch * 16) : kBufferOob;
+    }
+#pragma unroll
+    for (int d = 0; d < C::WD; ++d) {
+        const int q = (wave * C::WD + d) * 64 + lane, r = q / CHW, ch = swz<CHW>(r, q % CHW);
+        const int64_t n = weight_row<SWIGLU>(n0, gr.per, r, N);
+        wk0[d] = (C::FP8 ? 16 : 8) * ch;
+        woff[d] = n >= 0 ? (uint32_t)(n * K * (C::FP8 ? 1 : 2) + ch * 16) : kBufferOob;
+    }
+    const uint32_t m0x = __builtin_amdgcn_readfirstlane(lds0 + wave * C::XD * 1024);
+    const uint32_t m0w = __builtin_amdgcn_readfirstlane(lds0 + C::X_STAGE + wave * C::WD * 1024);
+    auto issue = [&](int t, uint32_t slot) __attribute__((always_inline)) {
+        // past the range's last step: nothing (the same number of DMAs)
+        const int k = (t0 + t) * C::BK, kend = t < KT ? K : 0;
+#pragma unroll
+        for (int d = 0; d < C::XD; ++d)
+            dma16(m0x + slot + d * 1024, k + xk[d] < kend ? xoff[d] : kBufferOob, dx, k * 2);
+#pragma unroll
+        for (int d = 0; d < C::WD; ++d)
+            dma16(m0w + slot + d * 1024, k + wk0[d] < kend ? woff[d] : kBufferOob, dw, C::FP8 ? k : k * 2);
+    };
+    // FP8: the tile's scales of this K range in fragment row order, [BN][stride].
+    float* sc = reinterpret_cast<float*>(smem + C::RING);
+    const int kb0 = S == 1 ? 0 : (t0 * C::BK) >> 7, SB = scale_blocks<C>(S, KT);
+    const int sstride = SB | 1;
+    if constexpr (C::FP8) {
+        for (int i = threadIdx.x; i < C::BN * SB; i += C::THREADS) {
+            const int r = i / SB, c = i - r * SB;
+            const int64_t n = weight_row<SWIGLU>(n0, gr.per, r, N);
+            sc[r * sstride + c] = n >= 0 && kb0 + c < S ? scales[n * S + kb0 + c] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < C::ST - 1; ++p) issue(p, p * C::STAGE);
+
+    f32x16 acc[C::MT][C::NT];
+#pragma unroll
+    for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+        for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    // Fragment row bases; the swizzle of a row depends on the row mod 16 only.
+    const uint32_t xrow = lds0 + (wm * (C::BM / C::WM) + l32) * C::XROW;
+    const uint32_t wrow = lds0 + C::X_STAGE + (wn * (C::BN / C::WN) + l32) * C::WROW;
+    const float* srow = sc + (wn * (C::BN / C::WN) + l32) * sstride;
+    // A slice of 32 K: lane half h holds K [16 h, 16 h + 16) of it, its first
+    // 8 in the first MFMA and the rest in the second, for x and W alike.
+    constexpr int SETS = C::PIPE ? 2 : 1;
+    u32x4 a[SETS][C::NT][2], b[SETS][C::MT][2], raw[C::NT];
+    float scl[C::NT];
+    auto fetch = [&](int set, uint32_t stage, int s, int t) __attribute__((always_inline)) {
+        if constexpr (C::FP8) {
+            const int kb = S == 1 ? 0 : min((((t0 + t) * C::BK) >> 7) - kb0, SB - 1);
+#pragma unroll
+            for (int j = 0; j < C::NT; ++j) {
+                raw[j] = lds16(wrow + stage + j * 32 * C::WROW + 16 * swz<CHW>(l32, 2 * s + h));
+                scl[j] = srow[j * 32 * sstride + kb];
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    a[set][j][e] = lds16(wrow + stage + j * 32 * C::WROW + 16 * swz<CHW>(l32, 4 * s + 2 * h + e));
+        }
+#pragma unroll
+        for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                b[set][i][e] = lds16(xrow + stage + i * 32 * C::XROW + 16 * swz<CHX>(l32, 4 * s + 2 * h + e));
+    };
+    auto convert = [&](int set) __attribute__((always_inline)) {
+        if constexpr (C::FP8) {
+#pragma unroll
+            for (int j = 0; j < C::NT; ++j) {
+                uint32_t o[8];
+                dequant4(raw[j].x, scl[j], o[0], o[1]);
+                dequant4(raw[j].y, scl[j], o[2], o[3]);
+                dequant4(raw[j].z, scl[j], o[4], o[5]);
+                dequant4(raw[j].w, scl[j], o[6], o[7]);
+                a[set][j][0] = u32x4{o[0], o[1], o[2], o[3]};
+                a[set][j][1] = u32x4{o[4], o[5], o[6], o[7]};
+            }
+        }
+    };
+    auto multiply = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+                for (int j = 0; j < C::NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[set][j][e]),
+                                                                        __builtin_bit_cast(bf16x8, b[set][i][e]),
+                                                                        acc[i][j], 0, 0, 0);
+    };
+    constexpr int SL = C::SLICES / C::WK;  // slices of a wave per step
+    uint32_t rd = 0, nx = C::STAGE, wr = (C::ST - 1) * C::STAGE;
+    auto next = [&](uint32_t v) __attribute__((always_inline)) { return v == (C::ST - 1) * C::STAGE ? 0u : v + C::STAGE; };
+    if constexpr (C::PIPE) {
+        static_assert(SL == 1 || SL % 2 == 0, "register sets alternate");
+        // Step t: stages t and t + 1 have landed for every wave, and every
+        // wave is done reading stage t - 1, whose slot takes stage t + ST - 1.
+        auto step = [&](int t, int p) __attribute__((always_inline)) {
+            wait_vm_barrier<(C::ST - 3) * C::ND>();
+            issue(t + C::ST - 1, wr);
+#pragma unroll
+            for (int s0 = 0; s0 < SL; ++s0) {
+                const int cur = (p + s0) & 1;
+                if (s0 + 1 < SL)
+                    fetch(cur ^ 1, rd, (s0 + 1) * C::WK + wk, t);
+                else
+                    fetch(cur ^ 1, nx, wk, t + 1);
+                multiply(cur);
+                convert(cur ^ 1);
+            }
+            rd = nx;
+            nx = next(nx);
+            wr = next(wr);
+        };
+        wait_vm_barrier<(C::ST - 2) * C::ND>();
+        fetch(0, rd, wk, 0);
+        convert(0);
+        if constexpr (SL == 1) {
+            for (int t = 0; t < KT; t += 2) {
+                step(t, 0);
+                if (t + 1 < KT) step(t + 1, 1);
+            }
+        } else {
+            for (int t = 0; t < KT; ++t) step(t, 0);
+        }
+    } else {
+        for (int t = 0; t < KT; ++t) {
+            wait_vm_barrier<(C::ST - 2) * C::ND>();
+            issue(t + C::ST - 1, wr);
+#pragma unroll
+            for (int s0 = 0; s0 < SL; ++s0) {
+                fetch(0, rd, s0 * C::WK + wk, t);
+                convert(0);
+                multiply(0);
+            }
+            rd = next(rd);
+            wr = next(wr);
+        }
+    }
+    // The last steps prefetched zeros past K; they must land before the ring
+    // is reused or the workgroup's LDS is freed.
+    wait_vm_barrier<0>();
+
+    if constexpr (C::WK > 1) {
+        // Wave (wk, q) leaves its tile at [q][fragment quad][lane]; wave (0, q)
+        // adds the partials in wk order, one wk at a time.
+        constexpr int Q = C::WM * C::WN, QUADS = C::MT * C::NT * 4;
+        f32x4* part = reinterpret_cast<f32x4*>(smem) + (wave % Q) * QUADS * 64 + lane;
+        for (int k = 1; k < C::WK; ++k) {
+            if (wk == k) {
+#pragma unroll
+                for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q)
+                            part[((i * C::NT + j) * 4 + q) * 64] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                                         acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+            }
+            __syncthreads();
+            if (wk == 0) {
+#pragma unroll
+                for (int i = 0; i < C::MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < C::NT; ++j)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const f32x4 p = part[((i * C::NT + j) * 4 + q) * 64];
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[i][j][4 * q + e] += p[e];
+                        }
+            }
+            if (k + 1 < C::WK) __syncthreads();
+        }
+        if (wk != 0) return;
+    }
+
+    // ---- epilogue: lane (h, l32) of fragment (i, j) holds row
+    // m0 + 32 (wm MT + i) + l32 and tile columns 32-block + 16 h + [0, 16)
+    // (SWIGLU: outputs 16-block + 8 h + [0, 8)).
+    constexpr int OW = SWIGLU ? 8 : 16;  // outputs of a lane and fragment
+    const int lim = min(n0 + gr.per, SWIGLU ? N >> 1 : N);
+#pragma unroll
+    for (int i = 0; i < C::MT; ++i) {
+        const int m = m0 + wm * (C::BM / C::WM) + 32 * i + l32;
+#pragma unroll
+        for (int j = 0; j < C::NT; ++j) {
+            const int col = n0 + (wn * C::NT + j) * 2 * OW + OW * h;
+            if (m >= M || col >= lim) continue;
+            if constexpr (!SWIGLU) {
+                if (gr.splits > 1) {
+                    float* dst = part + ((int64_t)split * M + m) * gr.ldp + col;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        if (col + 4 * q < lim)
+                            reinterpret_cast<f32x4*>(dst)[q] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1],
+                                                                     acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                    continue;
+                }
+            }
+            uint32_t o[OW / 2];
+            if constexpr (SWIGLU) {
+                uint32_t gu[8];
+                uint16_t v[8];
+#pragma unroll
+                for (int r = 0; r < 8; ++r) gu[r] = pack_bf16x2(f32x2{acc[i][j][r], acc[i][j][r + 8]});
+                swiglu_bf16_batch<8>(gu, v);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[r] = (uint32_t)v[2 * r] | ((uint32_t)v[2 * r + 1] << 16);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) o[r] = pack_bf16x2(f32x2{acc[i][j][2 * r], acc[i][j][2 * r + 1]});
+                if (bias) {
+                    add_bias8(o, bias, col, lim, gr.wide & 2);
+                    add_bias8(o + 4, bias, col + 8, lim, gr.wide & 2);
+                }
+            }
+            uint16_t* dst = y + (int64_t)m * ldy + col;
+#pragma unroll
+            for (int q = 0; q < OW / 8; ++q) {
+                if ((gr.wide & 1) && col + 8 * q + 8 <= lim) {
+                    reinterpret_cast<u32x4*>(dst)[q] = u32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
+                } else {
+#pragma unroll
+                    for (int r = 8 * q; r < 8 * q + 8; ++r)
+                        if (col + r < lim) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
+                }
+            }
+        }
+    }
+}
+
+// y = bf16(sum over splits, in order) (+ bias), or SWIGLU y = swiglu of the
+// gate and up sums: eight outputs per thread.
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part, int splits, int ldp,
+                                                           const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
+                                                           int64_t ldy, int M, int N, int wide) {
+    const int D = SWIGLU ? N >> 1 : N, groups = (D + 7) / 8;
+    const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (idx >= (int64_t)M * groups) return;
+    const int m = (int)(idx / groups), col = 8 * (int)(idx % groups);
+    const int64_t stride = (int64_t)M * ldp;
+    // D % 8 != 0: up's groups start off the 16-byte grid
+    auto sum8 = [&](int c, float (&v)[8]) __attribute__((always_inline)) {
+        const float* p = part + (int64_t)m * ldp + c;
+        if ((c & 3) == 0) {
+            f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
+            for (int s = 1; s < splits; ++s) {
+                a += *reinterpret_cast<const f32x4*>(p + s * stride);
+                b += *reinterpret_cast<const f32x4*>(p + s * stride + 4);
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = a[r], v[4 + r] = b[r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const int cc = c + r < N ? r : 0;
+                v[r] = p[cc];
+                for (int s = 1; s < splits; ++s) v[r] += p[s * stride + cc];
+            }
+        }
+    };
+    float a[8];
+    uint32_t o[4];
+    sum8(col, a);
+    if constexpr (SWIGLU) {
+        float b[8];
+        uint32_t gu[8];
+        uint16_t v[8];
+        sum8(D + col, b);
+#pragma unroll
+        for (int r = 0; r < 8; ++r) gu[r] = pack_bf16x2(f32x2{a[r], b[r]});
+        swiglu_bf16_batch<8>(gu, v);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = (uint32_t)v[2 * r] | ((uint32_t)v[2 * r + 1] << 16);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = pack_bf16x2(f32x2{a[2 * r], a[2 * r + 1]});
+        if (bias) add_bias8(o, bias, col, N, wide & 2);
+    }
+    uint16_t* dst = y + (int64_t)m * ldy + col;
+    if ((wide & 1) && col + 8 <= D) {
+        *reinterpret_cast<u32x4*>(dst) = u32x4{o[0], o[1], o[2], o[3]};
+    } else {
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+            if (col + r < D) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
+    }
+}
+
+inline hipError_t allow_lds(const void* kern, int bytes) {
+    return hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+}
+
+// The launch of config C over grid gr (part: splits > 1, gr.splits x M x
+// gr.ldp floats).
+template <class C, bool SWIGLU>
+hipError_t launch(const uint16_t* x, const void* w, const float* scales, int S, const uint16_t* bias, uint16_t* y,
+                  int64_t ldy, int M, int N, int K, const Grid& gr, float* part, hipStream_t stream) {
+    auto kern = gemm_tile_kernel<C, SWIGLU>;
+    static const hipError_t attr = allow_lds(reinterpret_cast<const void*>(kern), kLds);
+    if (attr != hipSuccess) return attr;
+    const int units = gr.mtiles * gr.nblocks * gr.splits;
+    hipLaunchKernelGGL(kern, dim3((unsigned)((units + 7) / 8 * 8)), dim3(C::THREADS), C::lds_bytes(S, K, gr.splits), stream,
+                       x, w, scales, S, bias, y, ldy, M, N, K, gr, part);
+    return hipGetLastError();
+}
+
+}  // namespace gemm_tile
+}  // namespace fp8lin

@@ -65,6 +65,25 @@ hipError_t launch_small_m_candidates(const uint16_t* x, const uint8_t* codes, co
 hipError_t launch_candidates_finish(const uint32_t* part, int M, int64_t chunks, int64_t offset, double* out,
                                     hipStream_t stream);
 
+// One-tile-per-workgroup GEMM (gemm_tile.hip) for BF16 weights or E4M3FN codes
+// (fp8) whose rows start on 16 bytes.  tile_plan picks tile and K ranges;
+// splits > 1 needs a 16-byte aligned workspace of tile_plan_bytes.  bias (or
+// null) is added to the rounded outputs; swiglu needs fp8.
+struct TilePlan {
+    int cfg, splits;
+    float us;  // estimated time
+};
+bool tile_supported(const uint16_t* x, const void* w, bool fp8, int S, int64_t M, int64_t N, int64_t K);
+TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split);
+size_t tile_plan_bytes(const TilePlan& p, int M, int N);
+hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,
+                       const uint16_t* bias, uint16_t* y, int64_t ldy, int M, int N, int K, bool swiglu, void* ws,
+                       hipStream_t stream);
+
+// BF16 weights: y = x * w^T (+ bias), M > 8 (gemm.hip).
+hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
+                            int N, int K, hipStream_t stream);
+
 // MFMA GEMM (gemm.hip).  B is E4M3FN codes (scales != nullptr, dequantized
 // to BF16 in LDS) or BF16 (scales == nullptr).  When swiglu, N is the number
 // of weight rows (gate rows [0,N/2), up rows [N/2,N)) and y is [M, N/2].

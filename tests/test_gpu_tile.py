@@ -1,0 +1,57 @@
+"""GPU parity of the one-tile-per-workgroup GEMM (csrc/gemm_tile.hpp) at the
+edges of its tiles: every tile of its table, rows and columns one past a tile
+edge, column counts off the 8- and 16-column store groups, K ending inside a
+slice, a step and a ring."""
+import numpy as np
+import pytest
+import torch
+
+from parity import assert_parity, bf16_to_f32
+from test_gpu_parity import bits, rand_bf16, up
+
+pytestmark = pytest.mark.gpu
+
+
+def sample(m):
+    """All rows of a small call, else the first, the tile edges and the last."""
+    return np.arange(m) if m <= 64 else np.unique(np.r_[0, 31, 32, 63, 64, 127, 128, m // 2, m - 2, m - 1].clip(0, m - 1))
+
+
+# One row per tile (32x32, 64x32, 64x64, 128x64, 128x128 with K over two
+# waves, 128x128 at two per CU, 256x256), then a shape with whole steps.
+@pytest.mark.parametrize("m,n,k", [(9, 261, 40), (515, 257, 1160), (33, 4100, 136), (9, 8200, 200), (65, 8195, 136),
+                                   (65, 17412, 200), (2050, 4100, 72), (2050, 2052, 136), (2050, 17412, 40),
+                                   (256, 2048, 512)])
+def test_bf16_tile(fp8lin, gpu, oracle, m, n, k):
+    """BF16 weights with a bias through the engine: the rows of the oracle's
+    product, the bias added to the rounded outputs, and no row touched by
+    another row's infinities."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    w, x, b = rand_bf16(rng, (n, k), 0.05), rand_bf16(rng, (m, k)), rand_bf16(rng, (n,))
+    y = fp8lin.gemm_bf16(up(x, gpu), up(w, gpu))
+    rows = sample(m)
+    assert_parity(bits(y)[rows], oracle.linear_bf16w(x[rows], w), f"bf16 tile {m}x{n}x{k}")
+    eng = fp8lin.LinearEngine()
+    eng.add("p.weight", up(w, gpu))
+    eng.add("p.bias", up(b, gpu))
+    assert torch.equal(eng.linear(up(x, gpu), "p"), fp8lin.add_bias(y.clone(), up(b, gpu)))
+    x[m // 2] = 0x7f80  # +inf
+    z = fp8lin.gemm_bf16(up(x, gpu), up(w, gpu))
+    keep = np.arange(m) != m // 2
+    assert torch.equal(z[keep], y[keep])
+    assert not np.isfinite(bf16_to_f32(bits(z)[m // 2])).any()
+
+
+def test_bf16_tile_output_stride_and_unaligned(fp8lin, gpu, oracle):
+    """A column slice of a wider output off the 16-byte grid (scalar stores),
+    and operands off it (the general kernel), give the aligned call's rows."""
+    rng = np.random.default_rng(5)
+    m, n, k = 70, 300, 264
+    w, x = rand_bf16(rng, (n, k), 0.05), rand_bf16(rng, (m, k))
+    ref = oracle.linear_bf16w(x, w)
+    wide = torch.zeros((m, n + 13), dtype=torch.bfloat16, device=gpu)
+    fp8lin.gemm_bf16(up(x, gpu), up(w, gpu), out=wide[:, 3:3 + n])
+    assert_parity(bits(wide[:, 3:3 + n]), ref, "strided output")
+    assert not wide[:, :3].any() and not wide[:, 3 + n:].any()
+    xs = torch.empty(m * k + 1, dtype=torch.bfloat16, device=gpu)[1:].view(m, k).copy_(up(x, gpu))
+    assert_parity(bits(fp8lin.gemm_bf16(xs, up(w, gpu))), ref, "unaligned x")
