@@ -148,11 +148,19 @@ size_t linear_ws(int64_t M, int64_t N, int64_t K, int64_t ldy) {
     return fp8lin::gemm_workspace_bytes((int)ceil_div(K, 128), ldy, (int)M, (int)N, (int)K, false);
 }
 
-// ws: the K-split partials of the prefill GEMM (linear_ws bytes), or null to
-// run every GEMM tile whole.
+// The part of a GEMM workspace that a call is refused without: the persistent
+// GEMM's split.  The tiles' partials, where the reported size holds them too,
+// are used when the caller brought that much and done without otherwise.
+size_t required_ws(int64_t S, int64_t ldy, int64_t M, int64_t N, int64_t K, bool swiglu) {
+    if (M <= 8 || M >= kMaxDim) return 0;
+    return fp8lin::gemm_split_bytes((int)S, ldy, (int)M, (int)N, (int)K, swiglu);
+}
+
+// ws: the K-split partials of the prefill GEMM (linear_ws bytes); may_split
+// false: run every GEMM tile whole.
 void linear_impl(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t S,
                  uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t stream,
-                 void* ws = nullptr, size_t ws_bytes = 0) {
+                 bool may_split = false, void* ws = nullptr, size_t ws_bytes = 0) {
     if (linear_small_m(x, codes, S, M, N, K)) {
         check_hip(fp8lin::launch_small_m(x, codes, scales, y, ldy, (int)M, (int)N, (int)K, 1, false, stream),
                   "fp8 small-M launch");
@@ -163,7 +171,7 @@ void linear_impl(const uint16_t* x, const uint8_t* codes, const float* scales, i
                   "fp8 gemv launch");
     } else {
         check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)S, y, ldy, (int)M, (int)N, (int)K, false,
-                                         ws_bytes ? ws : nullptr, ws_bytes, stream),
+                                         may_split, ws, ws_bytes, stream),
                   "fp8 gemm launch");
     }
 }
@@ -347,11 +355,11 @@ int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const 
     // :222-224
     if (w.scales && o.optimized && !(o.cublas_prefill && rows > 8)) {
         if (rows > 8) {
-            const size_t need = engine_gemm_ws(w, rows, ldy);
+            const size_t need = required_ws(w.scale_cols, ldy, rows, w.N, w.K, false);
             require(need == 0 || (ws != nullptr && ws_bytes >= need && aligned16(ws)), FP8LIN_ERR_WORKSPACE,
                     "FP8 GEMM split-K partial workspace missing, too small or unaligned");
             check_hip(fp8lin::launch_gemm_ws(x, codes, w.scales, (int)w.scale_cols, y, ldy, (int)rows, (int)w.N,
-                                             (int)w.K, false, need ? ws : nullptr, need, stream),
+                                             (int)w.K, false, true, ws, ws_bytes, stream),
                       "fp8 gemm launch");
         } else {
             linear_impl(x, codes, w.scales, w.scale_cols, y, ldy, rows, w.N, w.K, stream);
@@ -538,11 +546,10 @@ int fp8lin_linear_ws(const uint16_t* x, const uint8_t* codes, const float* scale
         require(x && codes && y, FP8LIN_ERR_ARGUMENT, "FP8 linear: null pointer");
         check_dims(M, N, K);
         check_scales(scales, scale_cols, K);
-        const size_t need = linear_ws(M, N, K, N);
-        check_workspace(workspace, workspace_bytes, need, "FP8 linear: workspace too small");
+        check_workspace(workspace, workspace_bytes, required_ws(ceil_div(K, 128), N, M, N, K, false),
+                        "FP8 linear: workspace too small");
         ensure_device();
-        linear_impl(x, codes, scales, scale_cols, y, N, M, N, K, as_stream(stream), need ? workspace : nullptr,
-                    need);
+        linear_impl(x, codes, scales, scale_cols, y, N, M, N, K, as_stream(stream), true, workspace, workspace_bytes);
     });
 }
 
@@ -558,8 +565,8 @@ int fp8lin_linear_swiglu(const uint16_t* x, const uint8_t* codes, const float* s
         if (M <= 8) {
             decode_swiglu(x, codes, scales, scale_cols, y, M, N, K, as_stream(stream));
         } else {
-            check_hip(fp8lin::launch_gemm(x, codes, scales, (int)scale_cols, y, N / 2, (int)M,
-                                          (int)N, (int)K, true, as_stream(stream)),
+            check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)scale_cols, y, N / 2, (int)M,
+                                             (int)N, (int)K, true, false, nullptr, 0, as_stream(stream)),
                       "fp8 gemm+swiglu launch");
         }
     });
@@ -590,14 +597,14 @@ int fp8lin_linear_swiglu_ws(const uint16_t* x, const uint8_t* codes, const float
         check_dims(M, N, K);
         require(N % 2 == 0, FP8LIN_ERR_SHAPE, "Invalid SwiGLU input: N must be even");
         check_scales(scales, scale_cols, K);
-        const size_t need = fp8lin_linear_swiglu_workspace_bytes(M, N, K);
-        check_workspace(workspace, workspace_bytes, need, "linear+SwiGLU: workspace too small");
+        check_workspace(workspace, workspace_bytes, required_ws(ceil_div(K, 128), N / 2, M, N, K, true),
+                        "linear+SwiGLU: workspace too small");
         ensure_device();
         if (M <= 8) {
             decode_swiglu(x, codes, scales, scale_cols, y, M, N, K, as_stream(stream));
         } else {
             check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)scale_cols, y, N / 2, (int)M, (int)N, (int)K,
-                                             true, need ? workspace : nullptr, need, as_stream(stream)),
+                                             true, true, workspace, workspace_bytes, as_stream(stream)),
                       "fp8 gemm+swiglu launch");
         }
     });

@@ -1,13 +1,8 @@
-// Prefill GEMM dispatch.  FP8 weights with K % 256 == 0 (every benchmark
-// shape) run gemm_fp8_kernel (gemm_fp8.hpp); other K, unaligned operands and
-// BF16 weights run the general template of gemm_kernel.hpp.
-//
-// General template, as measured on MI355X at the prefill shapes (M =
-// 512..4096, N = 17408, K = 5120, fused SwiGLU): a 256x256 workgroup tile of 8 waves
-// (2 along M x 4 along N, 128x64 per wave as 4x2 accumulators of
-// v_mfma_f32_32x32x16_bf16), K step 64, global loads issued two K steps ahead,
-// the next stage's FP8 dequantization and LDS store placed after the second
-// MFMA group, and the scheduler's MFMA/LDS interleave strategy 1.
+// Prefill GEMM dispatch.  FP8 weights with K % 256 == 0 run gemm_fp8_kernel
+// (gemm_fp8.hpp) or, where its estimate is lower, one tile per workgroup
+// (gemm_tile.hip); other K whose rows start on 16 bytes and BF16 weights run
+// the tiles, and what is left (unaligned operands, K off the 16-byte grid,
+// 2 GiB operands) the general template of gemm_kernel.hpp.
 #include <algorithm>
 #include <atomic>
 
@@ -18,17 +13,12 @@
 namespace fp8lin {
 namespace {
 
-using Tile = gemm::Cfg<256, 256, 64, 2, 4>;
-constexpr int kGroupM = 8;   // XCD-local tile patch height
-constexpr int kIglp = 1;     // MFMA / LDS interleave strategy
-constexpr int kPrefetch = 2; // global loads two K steps ahead
-constexpr int kStoreAt = 1;  // next-stage store after MFMA sub-step 1
+constexpr int kGroupM = 8;  // XCD-local tile patch height
 
 template <bool FP8, bool SWIGLU>
 hipError_t run(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y,
                int64_t ldy, int M, int N, int K, hipStream_t stream) {
-    return gemm::launch<Tile, FP8, SWIGLU, kGroupM, kIglp, kPrefetch, kStoreAt>(x, w, scales, S, y, ldy,
-                                                                             M, N, K, stream);
+    return gemm::launch<gemm::Cfg<256, 256, 64, 2, 4>, FP8, SWIGLU, kGroupM>(x, w, scales, S, y, ldy, M, N, K, stream);
 }
 
 // Work plan of the persistent FP8 GEMM (see gemm_fp8.hpp).  Without a
@@ -205,54 +195,87 @@ int compute_units() {
     return v;
 }
 
-size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu) {
-    if (skinny(M, N, swiglu) || mid_rows(nullptr, nullptr, S, M, N, K) ||
-        !fp8_kernel_ok(nullptr, nullptr, S, ldy, M, N, K))
+namespace {
+
+// Estimated us of the persistent FP8 GEMM under plan p, from its measured
+// times: 5.6 us per 256 K and round of 256-row tiles (6.5 where whole rounds
+// fill the chip and its clock falls), 4.1 of 128-row tiles, and for a split
+// the partials' round trip and the second launch.
+float estimate(const gemm_fp8::Plan& p, int K, int G) {
+    const int chunks = K / 256;
+    const float c = p.bm == 128 ? 4.1f : p.full >= G ? 6.5f : 5.6f;
+    float us = 5.0f + c * (float)(chunks * ((p.full + G - 1) / G));
+    if (p.rtiles > 0)
+        us += c * (float)((chunks + p.splits - 1) / p.splits) + 4.0f +
+              8.0e-6f / 6.0f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
+    return us;
+}
+
+// How an FP8 call of more than 8 rows that is neither skinny nor mid rows
+// runs: the persistent GEMM under `plan`, the tiles under `tile`, or (neither)
+// the general template.  have: the bytes of workspace that K-split partials
+// may take; a plan that needs more is made without a split.  The persistent
+// GEMM's unsplit sums do not depend on the row count or the tile height, and
+// the entry points that take no workspace (any false) keep them: there the
+// tiles only run the K that it does not.
+struct Route {
+    bool gemm, tiles;
+    gemm_fp8::Plan plan;
+    TilePlan tile;
+};
+
+Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, int K, bool swiglu, bool any, size_t have) {
+    Route r{fp8_kernel_ok(x, w, S, ldy, M, N, K), false, {}, {}};
+    const int G = compute_units();
+    auto fitting = [&](bool sw) {
+        const gemm_fp8::Plan p = make_plan(M, N, K, sw, G, any);
+        return plan_bytes(p) <= have ? p : make_plan(M, N, K, sw, G, false);
+    };
+    if (r.gemm) r.plan = fitting(swiglu);
+    if (tile_supported(x, w, true, S, M, N, K) && (!r.gemm || any)) {
+        r.tile = tile_plan(true, S, M, N, K, any);
+        if (tile_plan_bytes(r.tile, M, N) > have) r.tile = tile_plan(true, S, M, N, K, false);
+        // against the plain form's plan for both epilogues: one route for both
+        r.tiles = r.tile.cfg >= 0 && (!r.gemm || r.tile.us < 0.95f * estimate(fitting(false), K, G));
+    }
+    if (r.tiles) r.gemm = false;
+    return r;
+}
+
+}  // namespace
+
+size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu) {
+    if (skinny(M, N, swiglu) || mid_rows(nullptr, nullptr, S, M, N, K) || !fp8_kernel_ok(nullptr, nullptr, S, ldy, M, N, K))
         return 0;
     return plan_bytes(make_plan(M, N, K, swiglu, compute_units(), true));
 }
 
-hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,
-                          int M, int N, int K, bool swiglu, void* ws, size_t ws_bytes, hipStream_t stream) {
-    if (skinny(M, N, swiglu)) return launch_skinny(x, w, scales, S, y, ldy, M, N, K, swiglu, stream);
-    const bool fp8 = scales != nullptr;
-    if (fp8 && mid_rows(x, w, S, M, N, K))
-        return launch_small_m(x, static_cast<const uint8_t*>(w), scales, y, ldy, M, N, K, 1, swiglu, stream);
-    if (fp8 && fp8_kernel_ok(x, w, S, ldy, M, N, K)) {
-        const uint8_t* codes = static_cast<const uint8_t*>(w);
-        const int G = compute_units();
-        gemm_fp8::Plan plan = make_plan(M, N, K, swiglu, G, ws != nullptr);
-        if (plan_bytes(plan) > ws_bytes || reinterpret_cast<uintptr_t>(ws) % 16 != 0)
-            plan = make_plan(M, N, K, swiglu, G, false);
-        if (plan.rtiles == 0 && halves(x, w, S, M, N, K))
-            return launch_halves(x, codes, scales, y, ldy, M, N, K, swiglu, stream);
-        float* part = static_cast<float*>(ws);
-        return swiglu ? run_fp8<true>(x, codes, scales, S, y, ldy, M, N, K, plan, G, part, stream)
-                      : run_fp8<false>(x, codes, scales, S, y, ldy, M, N, K, plan, G, part, stream);
-    }
-    return launch_gemm(x, w, scales, S, y, ldy, M, N, K, swiglu, stream);
+size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu) {
+    if (skinny(M, N, swiglu) || mid_rows(nullptr, nullptr, S, M, N, K)) return 0;
+    const Route r = route(nullptr, nullptr, S, ldy, M, N, K, swiglu, true, SIZE_MAX);
+    const size_t gemm = gemm_split_bytes(S, ldy, M, N, K, swiglu);
+    return r.tiles ? std::max(gemm, tile_plan_bytes(r.tile, M, N)) : gemm;
 }
 
-hipError_t launch_gemm(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y,
-                       int64_t ldy, int M, int N, int K, bool swiglu, hipStream_t stream) {
+hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,
+                          int M, int N, int K, bool swiglu, bool may_split, void* ws, size_t ws_bytes,
+                          hipStream_t stream) {
     if (skinny(M, N, swiglu)) return launch_skinny(x, w, scales, S, y, ldy, M, N, K, swiglu, stream);
-    const bool fp8 = scales != nullptr;
-    if (fp8 && mid_rows(x, w, S, M, N, K))
-        return launch_small_m(x, static_cast<const uint8_t*>(w), scales, y, ldy, M, N, K, 1, swiglu, stream);
-    if (fp8 && halves(x, w, S, M, N, K))
-        return launch_halves(x, static_cast<const uint8_t*>(w), scales, y, ldy, M, N, K, swiglu, stream);
-    if (fp8 && fp8_kernel_ok(x, w, S, ldy, M, N, K)) {
-        const uint8_t* codes = static_cast<const uint8_t*>(w);
+    const uint8_t* codes = static_cast<const uint8_t*>(w);
+    if (mid_rows(x, w, S, M, N, K)) return launch_small_m(x, codes, scales, y, ldy, M, N, K, 1, swiglu, stream);
+    const size_t have = ws != nullptr && reinterpret_cast<uintptr_t>(ws) % 16 == 0 ? ws_bytes : 0;
+    const Route r = route(x, w, S, ldy, M, N, K, swiglu, may_split, have);
+    if (r.gemm && r.plan.rtiles == 0 && halves(x, w, S, M, N, K))
+        return launch_halves(x, codes, scales, y, ldy, M, N, K, swiglu, stream);
+    if (r.tiles) return launch_tile(r.tile, true, x, w, scales, S, nullptr, y, ldy, M, N, K, swiglu, ws, stream);
+    if (r.gemm) {
         const int G = compute_units();
-        const gemm_fp8::Plan plan = make_plan(M, N, K, swiglu, G, false);
-        return swiglu ? run_fp8<true>(x, codes, scales, S, y, ldy, M, N, K, plan, G, nullptr, stream)
-                      : run_fp8<false>(x, codes, scales, S, y, ldy, M, N, K, plan, G, nullptr, stream);
+        float* part = static_cast<float*>(ws);
+        return swiglu ? run_fp8<true>(x, codes, scales, S, y, ldy, M, N, K, r.plan, G, part, stream)
+                      : run_fp8<false>(x, codes, scales, S, y, ldy, M, N, K, r.plan, G, part, stream);
     }
-    if (fp8)
-        return swiglu ? run<true, true>(x, w, scales, S, y, ldy, M, N, K, stream)
-                      : run<true, false>(x, w, scales, S, y, ldy, M, N, K, stream);
-    return swiglu ? run<false, true>(x, w, nullptr, 1, y, ldy, M, N, K, stream)
-                  : run<false, false>(x, w, nullptr, 1, y, ldy, M, N, K, stream);
+    return swiglu ? run<true, true>(x, w, scales, S, y, ldy, M, N, K, stream)
+                  : run<true, false>(x, w, scales, S, y, ldy, M, N, K, stream);
 }
 
 hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
@@ -260,7 +283,8 @@ hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t
     if (!skinny(M, N, false) && tile_supported(x, w, false, 1, M, N, K))
         return launch_tile(tile_plan(false, 1, M, N, K, false), false, x, w, nullptr, 1, bias, y, ldy, M, N, K, false,
                            nullptr, stream);
-    const hipError_t e = launch_gemm(x, w, nullptr, 1, y, ldy, M, N, K, false, stream);
+    const hipError_t e = skinny(M, N, false) ? launch_skinny(x, w, nullptr, 1, y, ldy, M, N, K, false, stream)
+                                             : run<false, false>(x, w, nullptr, 1, y, ldy, M, N, K, stream);
     return e != hipSuccess || !bias ? e : launch_bias(y, ldy, bias, M, N, stream);
 }
 

@@ -34,6 +34,15 @@ constexpr Tile tile(int slots, float tau, float tau1) {
 // (31), 40 x 7168 x 5120 19.9 (22.3), 300 x 5120 x 5120 30.5 (35.8), 4096 x
 // 8192 x 8192 456 (355: the library's large tile is the better one).  The
 // 256x256-only kernel this replaced took 47, 46, 571 (K % 64 != 0), 159.
+// E4M3FN codes, M x N x K in us (before: the persistent GEMM or, at K % 256,
+// the general template): 93 x 17408 x 5120 40 (47), 93 x 5120 x 8704 25.7
+// (34.8), 200 x 7168 x 5120 33.6 (40.1), 512 x 2048 x 2048 11.9 (26.3), 320 x
+// 5120 x 3072 21.8 (33.7), 128 x 6000 x 1152 8.8 (20.2), 128 x 5000 x 4304
+// 21.6 (606, byte loads), row scales 27 x 8192 x 5120 14.3 (72.8).
+// What bounds them: at 128 rows or fewer the activations, which every
+// workgroup reads in full, share its 64 B/clk of DMA with the codes that come
+// from HBM (about 40 KB/us per CU against 29 for codes alone); above, LDS
+// reads and MFMA issue that one barrier per step does not let overlap fully.
 // Small tiles split a step's K over the waves of the workgroup, so that a
 // wave's tile stays deep enough for its LDS reads; FP8 tiles keep WM = 1 up
 // to 128 rows, where every code is dequantized once.
@@ -44,7 +53,7 @@ const Tile kBf16[] = {
     tile<Cfg<false, 128, 64, 2, 1, 4, 128, 3, false>, false>(1, 0.68f, 0.68f),
     tile<Cfg<false, 128, 128, 2, 2, 2, 64, 4, true>, false>(1, 0.98f, 0.98f),
     tile<Cfg<false, 128, 128, 2, 2, 1, 64, 2, false>, false>(2, 1.80f, 1.15f),
-    tile<Cfg<false, 256, 256, 2, 4, 1, 64, 2, false>, false>(1, 2.95f, 2.95f),
+    tile<Cfg<false, 256, 256, 2, 4, 1, 64, 2, false>, false>(1, 3.10f, 3.10f),
 };
 const Tile kFp8[] = {
     tile<Cfg<true, 32, 32, 1, 1, 4, 128, 8, false>, true>(1, 0.34f, 0.34f),
@@ -55,22 +64,28 @@ const Tile kFp8[] = {
     tile<Cfg<true, 64, 128, 1, 2, 4, 128, 4, false>, true>(1, 0.76f, 0.76f),
     tile<Cfg<true, 96, 192, 1, 6, 2, 64, 5, true>, true>(1, 1.37f, 1.37f),
     tile<Cfg<true, 128, 128, 1, 4, 2, 64, 5, true>, true>(1, 1.27f, 1.27f),
-    tile<Cfg<true, 256, 128, 2, 4, 1, 64, 3, true>, true>(1, 2.00f, 2.00f),
-    tile<Cfg<true, 256, 256, 2, 4, 1, 64, 2, false>, true>(1, 3.20f, 3.20f),
+    tile<Cfg<true, 128, 128, 1, 4, 1, 64, 2, false>, true>(2, 1.95f, 1.50f),
+    tile<Cfg<true, 256, 256, 2, 4, 1, 64, 2, false>, true>(1, 3.40f, 3.40f),
 };
 constexpr int kMaxTileSplits = 8;
 
 int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
-// Microseconds of tile t over M x N x K in `splits` K ranges: launch, first
-// loads and last stores; the rounds of workgroups, each over its K range; and
-// for a split the partials written and read back and the second launch.
-float estimate(const Tile& t, int M, int N, int K, int splits, int cus) {
+// Microseconds of tile t over M x N x K in `splits` K ranges: per round of
+// workgroups its first loads and last stores and its steps (a third of whose
+// time goes with the share of the chip that runs them), and for a split the
+// partials written and read back and the second launch.
+float estimate(const Tile& t, int S, int M, int N, int K, int splits, int cus) {
     const int64_t units = (int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
-    const int steps = ceil_div(ceil_div(K, 128), splits);
-    const bool single = units <= cus;
-    const float rounds = single ? 1.0f : (float)ceil_div(units, (int64_t)cus * t.slots);
-    const float us = 4.0f + rounds * (float)steps * (single ? t.tau1 : t.tau);
+    const float steps = (float)ceil_div(ceil_div(K, 128), splits), fixed = 2.0f + 6.0f * (float)(t.bm * t.bn) / 65536.0f;
+    const int slots = 2 * t.lds(S, K, splits) <= gemm_tile::kLds ? t.slots : 1;
+    const float tau = slots < t.slots ? t.tau1 : t.tau;
+    const int64_t whole = units / ((int64_t)cus * slots), rest = units - whole * cus * slots;
+    float us = 2.0f + (float)whole * (fixed + steps * tau);
+    if (rest > cus)
+        us += fixed + steps * tau;
+    else if (rest > 0)
+        us += fixed + steps * t.tau1 * (0.65f + 0.35f * (float)rest / (float)cus);
     return splits == 1 ? us : us + 4.0f + 8.0e-6f * (float)splits * (float)M * (float)N / 6.0f;
 }
 
@@ -85,6 +100,7 @@ Grid grid_of(const Tile& t, int M, int N, int64_t ldy, const uint16_t* y, const 
     g.group_m = 8;
     g.ldp = ceil_div(N, 8) * 8 + 8;
     g.wide = (ldy % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 ? 1 : 0) |
+             (ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 8 == 0 ? 4 : 0) |
              (reinterpret_cast<uintptr_t>(bias) % 16 == 0 ? 2 : 0);
     // One round: spread the columns evenly over the CUs.
     g.per = t.bn;
@@ -118,7 +134,7 @@ TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split) {
         const int most = may_split ? std::min(kMaxTileSplits, ceil_div(K, 128)) : 1;
         for (int s = 1; s <= most && (s == 1 || tiles * s <= cus); ++s) {
             if (t.lds(S, K, s) > gemm_tile::kLds) continue;
-            const float us = estimate(t, M, N, K, s, cus);
+            const float us = estimate(t, S, M, N, K, s, cus);
             if (best.cfg < 0 || us < best.us) best = {i, s, us};
         }
     }
@@ -126,7 +142,7 @@ TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split) {
 }
 
 size_t tile_plan_bytes(const TilePlan& p, int M, int N) {
-    return p.splits == 1 ? 0 : (size_t)p.splits * M * (ceil_div(N, 8) * 8 + 8) * sizeof(float);
+    return p.splits <= 1 ? 0 : (size_t)p.splits * M * (ceil_div(N, 8) * 8 + 8) * sizeof(float);
 }
 
 hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,

@@ -94,6 +94,25 @@ __device__ __forceinline__ void add_bias8(uint32_t* o, const uint16_t* __restric
                                  bf16_bits_to_f32(o[r] >> 16) + bf16_bits_to_f32(v[r] >> 16)});
 }
 
+// The first `left` (at most eight) of the outputs o to dst, in the widest
+// stores that dst's alignment allows (Grid::wide).
+__device__ __forceinline__ void store8(uint16_t* dst, const uint32_t* o, int left, int wide) {
+    if ((wide & 1) && left >= 8) {
+        *reinterpret_cast<u32x4*>(dst) = u32x4{o[0], o[1], o[2], o[3]};
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        if ((wide & 4) && left >= 4 * q + 4) {
+            *reinterpret_cast<u32x2*>(dst + 4 * q) = u32x2{o[2 * q], o[2 * q + 1]};
+        } else {
+#pragma unroll
+            for (int r = 4 * q; r < 4 * q + 4; ++r)
+                if (r < left) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
+        }
+    }
+}
+
 // Position of chunk ch of row r in a row of CH chunks.
 template <int CH>
 __device__ __forceinline__ int swz(int r, int ch) {
@@ -143,7 +162,7 @@ struct Grid {
     int mtiles, nblocks, per, splits;
     int group_m;  // tile rows walked together (x and W rows shared in an XCD's L2)
     int ldp;      // row stride of the partials
-    int wide;     // 1: y rows hold 16-byte aligned 8-column groups; 2: so does bias
+    int wide;     // y's 8-column groups start on 16 bytes (1) or 8 (4); bias's on 16 (2)
 };
 
 // Requirements (checked by the launcher): x, w 16-byte aligned; K % 8 == 0
@@ -416,15 +435,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
             }
             uint16_t* dst = y + (int64_t)m * ldy + col;
 #pragma unroll
-            for (int q = 0; q < OW / 8; ++q) {
-                if ((gr.wide & 1) && col + 8 * q + 8 <= lim) {
-                    reinterpret_cast<u32x4*>(dst)[q] = u32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
-                } else {
-#pragma unroll
-                    for (int r = 8 * q; r < 8 * q + 8; ++r)
-                        if (col + r < lim) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
-                }
-            }
+            for (int q = 0; q < OW / 8; ++q) store8(dst + 8 * q, o + 4 * q, lim - col - 8 * q, gr.wide);
         }
     }
 }
@@ -479,13 +490,7 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
         if (bias) add_bias8(o, bias, col, N, wide & 2);
     }
     uint16_t* dst = y + (int64_t)m * ldy + col;
-    if ((wide & 1) && col + 8 <= D) {
-        *reinterpret_cast<u32x4*>(dst) = u32x4{o[0], o[1], o[2], o[3]};
-    } else {
-#pragma unroll
-        for (int r = 0; r < 8; ++r)
-            if (col + r < D) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
-    }
+    store8(dst, o, D - col, wide);
 }
 
 inline hipError_t allow_lds(const void* kern, int bytes) {

@@ -84,23 +84,21 @@ hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const voi
 hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
                             int N, int K, hipStream_t stream);
 
-// MFMA GEMM (gemm.hip).  B is E4M3FN codes (scales != nullptr, dequantized
-// to BF16 in LDS) or BF16 (scales == nullptr).  When swiglu, N is the number
-// of weight rows (gate rows [0,N/2), up rows [N/2,N)) and y is [M, N/2].
-hipError_t launch_gemm(const uint16_t* x, const void* w, const float* scales, int S,
-                       uint16_t* y, int64_t ldy, int M, int N, int K, bool swiglu,
-                       hipStream_t stream);
-// The FP8 GEMM with a workspace for K-split partials: where the tile count
-// leaves CUs idle (few tiles, or a small last round) K is split and a second
-// launch adds the FP32 partials.  gemm_workspace_bytes() is what that needs
-// (0 when nothing splits); a smaller or unaligned workspace, unaligned x or
-// w, or another kernel's shape run unsplit.
+// FP8 prefill GEMM (gemm.hip), M > 8, with a workspace for K-split partials
+// (or null; may_split false: an entry point that takes none): where whole tiles leave CUs idle K is split and a second launch
+// adds the FP32 partials.  gemm_workspace_bytes() is what the plan needs (0
+// when nothing splits); gemm_split_bytes() is the persistent GEMM's own part
+// of it.  A smaller or unaligned workspace, unaligned x or w, or another
+// kernel's shape run unsplit.  When swiglu, N is the number of weight rows
+// (gate rows [0,N/2), up rows [N/2,N)) and y is [M, N/2].
 size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
+size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 // Whether the GEMM dispatch sends this FP8 call (9..32 rows) to the small-M
 // matrix-core kernel instead of a GEMM tile.
 bool gemm_mid_rows(const uint16_t* x, const void* w, int S, int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,
-                          int M, int N, int K, bool swiglu, void* ws, size_t ws_bytes, hipStream_t stream);
+                          int M, int N, int K, bool swiglu, bool may_split, void* ws, size_t ws_bytes,
+                          hipStream_t stream);
 
 // Elementwise kernels (elementwise.hip).
 hipError_t launch_dequant(const uint8_t* codes, const float* scales, int64_t S, uint16_t* y,

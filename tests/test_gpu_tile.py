@@ -55,3 +55,55 @@ def test_bf16_tile_output_stride_and_unaligned(fp8lin, gpu, oracle):
     assert not wide[:, :3].any() and not wide[:, 3 + n:].any()
     xs = torch.empty(m * k + 1, dtype=torch.bfloat16, device=gpu)[1:].view(m, k).copy_(up(x, gpu))
     assert_parity(bits(fp8lin.gemm_bf16(xs, up(w, gpu))), ref, "unaligned x")
+
+
+# The FP8 tiles (32x32, 64x32, 64x64, 96x64, 128x64, 64x128, 96x192, 128x128
+# with K over two waves and at two per CU, 256x256) and K ranges of unequal
+# length.  K % 256 != 0 keeps the calls off the persistent GEMM.
+FP8_TILES = [(9, 261, 48), (70, 1030, 1168), (40, 4100, 400), (70, 4100, 144), (100, 8195, 272), (96, 16000, 144),
+             (33, 17412, 144), (129, 17412, 48), (520, 4096, 1168), (513, 8195, 144), (1030, 12290, 144), (9, 261, 4112),
+             (65, 4100, 4112)]
+
+
+@pytest.mark.parametrize("m,n,k", FP8_TILES)
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_tile(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """Block and row scales against the oracle on a sample of rows; the fused
+    SwiGLU equal to SwiGLU of the plain form, with and without a workspace; a
+    split only reorders sums."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random(n if rows_scaled else (n, (k + 127) // 128)) * .01 + .001).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    rows = sample(m)
+    ref = oracle.linear(x[rows], codes, scales)
+    for split in (False, True):
+        y = fp8lin.fp8_linear(xd, cd, sd, split=split)
+        assert_parity(bits(y)[rows], ref, f"fp8 tile {m}x{n}x{k} split={split}")
+        if n % 2 == 0:
+            assert torch.equal(fp8lin.linear_swiglu(xd, cd, sd, split=split), fp8lin.fused_swiglu(y))
+
+
+@pytest.mark.parametrize("m,n,k", [(70, 4096, 2048), (93, 5120, 3072), (129, 2048, 1024), (200, 1536, 4096),
+                                   (320, 2048, 2048), (513, 1030, 1280), (65, 17408, 4096)])
+def test_fp8_tile_beside_persistent_gemm(fp8lin, gpu, oracle, m, n, k):
+    """K the persistent GEMM takes too: with a workspace the tiles may run the
+    call, whole or in K ranges; the same product as the persistent GEMM's to
+    the parity bar, whatever workspace is brought."""
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random((n, k // 128)) * .01 + .001).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    rows = sample(m)
+    ref = oracle.linear(x[rows], codes, scales)
+    whole = fp8lin.fp8_linear(xd, cd, sd, split=False)
+    split = fp8lin.fp8_linear(xd, cd, sd)
+    assert_parity(bits(whole)[rows], ref, f"whole {m}x{n}x{k}")
+    assert_parity(bits(split)[rows], ref, f"split {m}x{n}x{k}")
+    assert torch.equal(split, fp8lin.fp8_linear(xd, cd, sd))
+    x[m // 2] = 0x7fc0  # NaN
+    bad = fp8lin.fp8_linear(up(x, gpu), cd, sd)
+    keep = np.arange(m) != m // 2
+    assert torch.equal(bad[keep], split[keep]) and torch.isnan(bad[m // 2]).all()
