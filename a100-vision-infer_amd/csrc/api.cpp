@@ -157,10 +157,12 @@ size_t required_ws(int64_t S, int64_t ldy, int64_t M, int64_t N, int64_t K, bool
 }
 
 // ws: the K-split partials of the prefill GEMM (linear_ws bytes); may_split
-// false: run every GEMM tile whole.
+// false: run every GEMM tile whole.  bias: added by the kernels that can, which
+// then set *bias_added.
 void linear_impl(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t S,
                  uint16_t* y, int64_t ldy, int64_t M, int64_t N, int64_t K, hipStream_t stream,
-                 bool may_split = false, void* ws = nullptr, size_t ws_bytes = 0) {
+                 bool may_split = false, void* ws = nullptr, size_t ws_bytes = 0, const uint16_t* bias = nullptr,
+                 bool* bias_added = nullptr) {
     if (linear_small_m(x, codes, S, M, N, K)) {
         check_hip(fp8lin::launch_small_m(x, codes, scales, y, ldy, (int)M, (int)N, (int)K, 1, false, stream),
                   "fp8 small-M launch");
@@ -171,7 +173,7 @@ void linear_impl(const uint16_t* x, const uint8_t* codes, const float* scales, i
                   "fp8 gemv launch");
     } else {
         check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)S, y, ldy, (int)M, (int)N, (int)K, false,
-                                         may_split, ws, ws_bytes, stream),
+                                         may_split, ws, ws_bytes, bias, bias_added, stream),
                   "fp8 gemm launch");
     }
 }
@@ -287,7 +289,7 @@ size_t engine_ws(const fp8lin_linear_options& o, const fp8lin_weight& w, int64_t
     if (w.cached_bf16 && rows > 1) return 0;
     // (the plan for ldy = N: a wider ldy never needs more)
     if (w.scales && o.optimized && !(o.cublas_prefill && rows > 8)) return engine_gemm_ws(w, rows, w.N);
-    if (w.scales) return dequant_gemm_ws(w.N, w.K);
+    if (w.scales) return std::max(dequant_gemm_ws(w.N, w.K), engine_gemm_ws(w, rows, w.N));
     return 0;
 }
 
@@ -358,28 +360,22 @@ int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const 
             const size_t need = required_ws(w.scale_cols, ldy, rows, w.N, w.K, false);
             require(need == 0 || (ws != nullptr && ws_bytes >= need && aligned16(ws)), FP8LIN_ERR_WORKSPACE,
                     "FP8 GEMM split-K partial workspace missing, too small or unaligned");
-            check_hip(fp8lin::launch_gemm_ws(x, codes, w.scales, (int)w.scale_cols, y, ldy, (int)rows, (int)w.N,
-                                             (int)w.K, false, true, ws, ws_bytes, stream),
-                      "fp8 gemm launch");
-        } else {
-            linear_impl(x, codes, w.scales, w.scale_cols, y, ldy, rows, w.N, w.K, stream);
         }
+        linear_impl(x, codes, w.scales, w.scale_cols, y, ldy, rows, w.N, w.K, stream, true, ws, ws_bytes, w.bias,
+                    &bias_added);
         return rows <= 8 ? FP8LIN_PATH_FP8_GEMV : FP8LIN_PATH_FP8_GEMM;
     }
-    // :225-233, 2048-row BF16 slabs, each GEMM writing its column slice of y.
+    // :225-233: dequantize, then GEMM.  The weight of that product is
+    // bf16(decode(c) * s), the value every FP8 kernel here multiplies with, so
+    // the FP8 kernels give it without a BF16 copy of the weight.  Slabs of
+    // 2048 rows, each a dequantization and a GEMM of 8 column tiles, took 1640
+    // us for 640 x 17408 x 5120, where the FP8 GEMM takes 122.
     if (w.scales) {
         const size_t need = dequant_gemm_ws(w.N, w.K);
         require(ws != nullptr && ws_bytes >= need && aligned16(ws), FP8LIN_ERR_WORKSPACE,
                 "dequant-then-GEMM slab workspace missing, too small or unaligned");
-        auto* slab = static_cast<uint16_t*>(ws);
-        for (int64_t begin = 0; begin < w.N; begin += kSlabRows) {
-            const int64_t count = w.N - begin < kSlabRows ? w.N - begin : kSlabRows;
-            const float* s = w.scales + begin * w.scale_cols;
-            check_hip(fp8lin::launch_dequant(codes + begin * w.K, s, w.scale_cols, slab, w.K, count,
-                                             w.K, stream),
-                      "dequant launch");
-            gemm_bf16_impl(x, slab, nullptr, y + begin, ldy, rows, count, w.K, stream);
-        }
+        linear_impl(x, codes, w.scales, w.scale_cols, y, ldy, rows, w.N, w.K, stream, true, ws, ws_bytes, w.bias,
+                    &bias_added);
         return FP8LIN_PATH_DEQUANT_GEMM;
     }
     // :234-237
@@ -566,7 +562,7 @@ int fp8lin_linear_swiglu(const uint16_t* x, const uint8_t* codes, const float* s
             decode_swiglu(x, codes, scales, scale_cols, y, M, N, K, as_stream(stream));
         } else {
             check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)scale_cols, y, N / 2, (int)M,
-                                             (int)N, (int)K, true, false, nullptr, 0, as_stream(stream)),
+                                             (int)N, (int)K, true, false, nullptr, 0, nullptr, nullptr, as_stream(stream)),
                       "fp8 gemm+swiglu launch");
         }
     });
@@ -604,7 +600,8 @@ int fp8lin_linear_swiglu_ws(const uint16_t* x, const uint8_t* codes, const float
             decode_swiglu(x, codes, scales, scale_cols, y, M, N, K, as_stream(stream));
         } else {
             check_hip(fp8lin::launch_gemm_ws(x, codes, scales, (int)scale_cols, y, N / 2, (int)M, (int)N, (int)K,
-                                             true, true, workspace, workspace_bytes, as_stream(stream)),
+                                             true, true, workspace, workspace_bytes, nullptr, nullptr,
+                                             as_stream(stream)),
                       "fp8 gemm+swiglu launch");
         }
     });

@@ -259,7 +259,7 @@ size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu
 
 hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,
                           int M, int N, int K, bool swiglu, bool may_split, void* ws, size_t ws_bytes,
-                          hipStream_t stream) {
+                          const uint16_t* bias, bool* bias_added, hipStream_t stream) {
     if (skinny(M, N, swiglu)) return launch_skinny(x, w, scales, S, y, ldy, M, N, K, swiglu, stream);
     const uint8_t* codes = static_cast<const uint8_t*>(w);
     if (mid_rows(x, w, S, M, N, K)) return launch_small_m(x, codes, scales, y, ldy, M, N, K, 1, swiglu, stream);
@@ -267,7 +267,10 @@ hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales,
     const Route r = route(x, w, S, ldy, M, N, K, swiglu, may_split, have);
     if (r.gemm && r.plan.rtiles == 0 && halves(x, w, S, M, N, K))
         return launch_halves(x, codes, scales, y, ldy, M, N, K, swiglu, stream);
-    if (r.tiles) return launch_tile(r.tile, true, x, w, scales, S, nullptr, y, ldy, M, N, K, swiglu, ws, stream);
+    if (r.tiles) {
+        if (bias) *bias_added = true;
+        return launch_tile(r.tile, true, x, w, scales, S, bias, y, ldy, M, N, K, swiglu, ws, stream);
+    }
     if (r.gemm) {
         const int G = compute_units();
         float* part = static_cast<float*>(ws);

@@ -89,7 +89,8 @@ hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t
 // adds the FP32 partials.  gemm_workspace_bytes() is what the plan needs (0
 // when nothing splits); gemm_split_bytes() is the persistent GEMM's own part
 // of it.  A smaller or unaligned workspace, unaligned x or w, or another
-// kernel's shape run unsplit.  When swiglu, N is the number of weight rows
+// kernel's shape run unsplit.  The tiles add bias (or null) and set
+// *bias_added; the other kernels leave it to the caller.  When swiglu, N is the number of weight rows
 // (gate rows [0,N/2), up rows [N/2,N)) and y is [M, N/2].
 size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
@@ -98,7 +99,7 @@ size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 bool gemm_mid_rows(const uint16_t* x, const void* w, int S, int64_t M, int64_t N, int64_t K);
 hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,
                           int M, int N, int K, bool swiglu, bool may_split, void* ws, size_t ws_bytes,
-                          hipStream_t stream);
+                          const uint16_t* bias, bool* bias_added, hipStream_t stream);
 
 // Elementwise kernels (elementwise.hip).
 hipError_t launch_dequant(const uint8_t* codes, const float* scales, int64_t S, uint16_t* y,

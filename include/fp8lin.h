@@ -219,8 +219,8 @@ int fp8lin_gemm_bf16(const uint16_t* x, const uint16_t* w, uint16_t* y, int64_t 
  * order is the reference's: tensor-small (rows 2..8, K%128==0, block scales;
  * tilelang_fp8 additionally N%16==0) -> multi-token shared GEMV (rows 2..8)
  * -> cached BF16 GEMM (rows > 1) -> fp8_linear (optimized, unless
- * cublas_prefill and rows > 8) -> dequant-then-GEMM in 2048-row slabs
- * (src/engine.cpp:225-233) -> BF16 GEMM for unquantized weights.  Then, when
+ * cublas_prefill and rows > 8) -> dequantized GEMM
+ * (src/engine.cpp:225-233; the FP8 kernels, whose weights are the dequantized values) -> BF16 GEMM for unquantized weights.  Then, when
  * the weight has a bias, y = bf16(y + bias) (src/engine.cpp:240).
  * The tensor-parallel reduce that the reference runs between the product and
  * the bias (src/engine.cpp:239) is the caller's: for a weight whose output is
@@ -257,8 +257,10 @@ typedef struct fp8lin_linear_options {
 /* Workspace needed by fp8lin_engine_linear for this weight and row count;
  * 0 if none.  The FP8 GEMM branch (rows > 8) splits K where its 256x256
  * tiles would leave CUs idle (as fp8lin_linear_swiglu_ws does) and then needs
- * 256 KiB of FP32 partials per split tile and K range; the dequant-then-GEMM
- * branch needs a 2048-row BF16 slab. */
+ * 256 KiB of FP32 partials per split tile and K range, or splits smaller
+ * tiles with rows x N partials per range (used when the workspace holds them);
+ * the dequantized-GEMM branch is refused with less than a 2048-row BF16 slab,
+ * the reference's, and splits in it. */
 size_t fp8lin_engine_linear_workspace_bytes(const fp8lin_linear_options* options,
                                             const fp8lin_weight* weight, int64_t rows);
 /* Id of the branch fp8lin_engine_linear takes for this weight, options and
