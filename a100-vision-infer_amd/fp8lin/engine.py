@@ -15,7 +15,7 @@ import ctypes
 
 import torch
 
-from ._lib import (ERR_ARGUMENT, PATH_TENSOR_SMALL, Fp8linError, LinearOptions, Weight, check, lib)
+from ._lib import (ERR_ARGUMENT, PATH_FP8_GEMM, PATH_FP8_GEMV, PATH_TENSOR_SMALL, Fp8linError, LinearOptions, Weight, check, lib)
 from .ops import fp8_decode, fused_swiglu, qk_norm_rope
 
 
@@ -221,13 +221,13 @@ class LinearEngine:
 
     def mlp(self, n, prefix):
         """The MLP of `Engine::step` (src/engine.cpp:415-416) on one rank:
-        optimized, `fused_swiglu(linear(n, gate_up))`; otherwise the unfused
+        optimized, `fused_swiglu(linear(n, gate_up))` (_linear_swiglu); otherwise the unfused
         `silu(linear(n, gate_proj)) * linear(n, up_proj)` on the source
         weights, with the same two BF16 rounding points (the SwiGLU of the two
         outputs side by side).  Then `linear(gated, down_proj)`; the
         cross-rank reduce is the caller's."""
         if self.options.optimized:
-            gated = fused_swiglu(self.linear(n, prefix + ".gate_up"))
+            gated = self._linear_swiglu(n, prefix + ".gate_up")
         else:
             gate = self.linear(n, prefix + ".gate_proj")
             up = self.linear(n, prefix + ".up_proj")
@@ -235,6 +235,28 @@ class LinearEngine:
             pair = torch.cat([gate.reshape(rows, -1), up.reshape(rows, -1)], -1)
             gated = fused_swiglu(pair).reshape(*gate.shape)
         return self.linear(gated, prefix + ".down_proj")
+
+    def _linear_swiglu(self, n, name):
+        """fused_swiglu(linear(n, name)): one launch (fp8lin_linear_swiglu_ws)
+        where `linear` would run its FP8 kernels on a weight without a bias,
+        with their sums and the two BF16 rounding points.  The separate pass
+        wrote and read the [rows, N] product: 80 of 940 us of an MLP at 3913
+        rows, a launch of 4 us at one row.  Other branches, and profiled calls
+        (whose events time the projections alone), keep the two calls."""
+        if n.dim() == 2 and not self.profile_kernels and name not in self.mixed_projections:
+            rec = self._record(name)
+            rows = n.size(0)
+            if not rec.bias and rec.N % 2 == 0 and lib().fp8lin_engine_linear_path(
+                    ctypes.byref(self.options), ctypes.byref(rec), rows) in (PATH_FP8_GEMV, PATH_FP8_GEMM):
+                x = n.contiguous()
+                y = torch.empty((rows, rec.N // 2), dtype=torch.bfloat16, device=n.device)
+                need = lib().fp8lin_linear_swiglu_workspace_bytes(rows, rec.N, rec.K)
+                ws = self._ws(need, n.device)
+                check(lib().fp8lin_linear_swiglu_ws(
+                    x.data_ptr(), rec.data, rec.scales, rec.scale_cols, y.data_ptr(), rows, rec.N, rec.K,
+                    ws.data_ptr() if ws is not None else None, need, torch.cuda.current_stream(n.device).cuda_stream))
+                return y
+        return fused_swiglu(self.linear(n, name))
 
     # -- dispatch --------------------------------------------------------------
     def _record(self, name):

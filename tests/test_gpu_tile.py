@@ -107,3 +107,31 @@ def test_fp8_tile_beside_persistent_gemm(fp8lin, gpu, oracle, m, n, k):
     bad = fp8lin.fp8_linear(up(x, gpu), cd, sd)
     keep = np.arange(m) != m // 2
     assert torch.equal(bad[keep], split[keep]) and torch.isnan(bad[m // 2]).all()
+
+
+@pytest.mark.parametrize("m", [1, 4, 27, 70, 300])
+@pytest.mark.parametrize("option", ["plain", "bias", "cached", "dequant", "profiled"])
+def test_engine_mlp_swiglu_forms(fp8lin, gpu, oracle, m, option):
+    """LinearEngine.mlp's gate/up, one launch or two: SwiGLU of the engine's
+    own product within one ulp where a split reorders sums, else bit for bit;
+    three-dimensional inputs stay refused."""
+    rng = np.random.default_rng(m)
+    d, k = 1040, 1024
+    eng = fp8lin.LinearEngine(fp8lin.LinearOptions(cublas_prefill=option == "dequant"), profile_kernels=option == "profiled",
+                              weight_cache_bytes=1 << 30 if option == "cached" else 0)
+    for name, rows, cols in (("l.gate_up", 2 * d, k), ("l.down_proj", 512, d - 16)):
+        codes, scales = fp8lin.gen_weights(rows, cols, seed=3, tag=rows, device=gpu)
+        eng.add(name + ".weight", codes, scales)
+    if option == "bias":
+        eng.add("l.gate_up.bias", up(rand_bf16(rng, (2 * d,)), gpu))
+    if option == "cached":
+        eng.build_cache()
+    x = up(rand_bf16(rng, (m, k)), gpu)
+    ref = fp8lin.fused_swiglu(eng.linear(x, "l.gate_up"))
+    got = eng._linear_swiglu(x, "l.gate_up")
+    if m in (70, 300):
+        assert_parity(bits(got), bits(ref), f"mlp {option} m={m}")
+    else:
+        assert torch.equal(got, ref)
+    with pytest.raises(fp8lin.Fp8linError):
+        eng._linear_swiglu(x[None], "l.gate_up")
