@@ -198,16 +198,16 @@ int compute_units() {
 namespace {
 
 // Estimated us of the persistent FP8 GEMM under plan p, from its measured
-// times: 5.6 us per 256 K and round of 256-row tiles (6.5 where whole rounds
-// fill the chip and its clock falls), 4.1 of 128-row tiles, and for a split
+// times: 4.8 us per 256 K and round of 256-row tiles (6.1 where whole rounds
+// fill the chip and its clock falls), 3.8 of 128-row tiles, and for a split
 // the partials' round trip and the second launch.
 float estimate(const gemm_fp8::Plan& p, int K, int G) {
     const int chunks = K / 256;
-    const float c = p.bm == 128 ? 4.1f : p.full >= G ? 6.5f : 5.6f;
+    const float c = p.bm == 128 ? 3.8f : p.full >= G ? 6.1f : 4.8f;
     float us = 5.0f + c * (float)(chunks * ((p.full + G - 1) / G));
     if (p.rtiles > 0)
         us += c * (float)((chunks + p.splits - 1) / p.splits) + 4.0f +
-              8.0e-6f / 6.0f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
+              8.0e-6f / 5.2f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
     return us;
 }
 

@@ -18,10 +18,11 @@
 //     256 x 128 B; the 16-byte chunks of a row are XOR-swizzled (ga) so the
 //     16 rows read by a quarter-wave of a fragment load hit distinct banks.
 //     All 4 waves share it; one barrier per step, in the middle of the step.
-//   B (FP8 codes): each wave DMAs its own 64 rows x 64 B per step (16 rows x
-//     64 B per instruction) into a private 3-slot LDS ring (swizzle gb), reads
-//     them back in the MFMA B-operand layout and dequantizes them in registers
-//     one step ahead.  No B data crosses waves, so B needs no barrier.
+//   B (FP8 codes): each wave DMAs its own 64 rows x 128 B every two steps (8
+//     rows x 128 B per instruction: 64-byte pieces read HBM slower) into one
+//     of two private LDS slots (swizzle ga) up to four steps ahead, reads them
+//     back in the MFMA B-operand layout and dequantizes them in registers one
+//     step ahead.  No B data crosses waves, so B needs no barrier.
 //   Scales: one dword per lane per 128-K block, loaded a step ahead.
 // The K index within a step is permuted identically for A and B (lane half h
 // of sub-step s covers k = 32*(s/2) + 16h + 8*(s%2) + [0,8)), which changes
@@ -47,8 +48,8 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 constexpr int WN = 64, BN = 256, BK = 64;
 constexpr int NT = 2;
 constexpr int THREADS = 256;
-constexpr int B_SLOT = WN * 64;  // 4 KiB: 64 rows x 64 codes
-constexpr int B_WAVE = 3 * B_SLOT;
+constexpr int B_SLOT = WN * 128;  // 8 KiB: 64 rows x 128 codes, two steps
+constexpr int B_WAVE = 2 * B_SLOT;
 
 // The tile's M extent: MT fragments of 32 rows.  MT = 8 (256 rows) is the
 // tile described above; MT = 4 (128 rows) serves launches of M <= 128 rows,
@@ -61,17 +62,23 @@ struct Geo {
     static constexpr int BM = 32 * MT;
     static constexpr int A_STAGE = BM * 128;  // BM rows x 64 BF16
     static constexpr int A_BYTES = 3 * A_STAGE;
-    static constexpr int LDS_BYTES = A_BYTES + 4 * B_WAVE;  // 144 KiB (MT 8) or 96 KiB (MT 4)
+    static constexpr int LDS_BYTES = A_BYTES + 4 * B_WAVE;  // 160 KiB (MT 8) or 112 KiB (MT 4)
     static constexpr int SLOT_FLOATS = BM * BN;             // one split partial
     static constexpr int MFMAS = 2 * MT;                    // per sub-step
     static constexpr int DQ = 16 / MT;                      // dequant instructions per MFMA
-    // Sub-step-0 slots of the 4 B DMAs (the 2 scale loads of odd steps sit
-    // in slots MT + 1 and MT + 3, after that slot's DMA).
-    static constexpr bool b_dma_at(int m) { return MT >= 8 ? (m >= MT && ((m - MT) & 1) == 0) : m >= MT; }
-    static constexpr int b_dma_index(int m) { return MT >= 8 ? (m - MT) >> 1 : m - MT; }
-    // Vector-memory operations issued after a step's last scale load: the
-    // B DMAs in later slots of sub-step 0 and the MT A DMAs of sub-step 2.
-    static constexpr int VM_AFTER_SCALE = (MT >= 8 ? 2 : 0) + MT;
+    // The 8 B DMAs of an even step are spread over its sub-step 3, after the
+    // step's A DMAs.  Vector-memory operations retire in order, so the next
+    // step's mid-step wait for those A DMAs also waits for all that was issued
+    // before them: behind the A DMAs the codes have until the mid-step wait
+    // after that.  Ahead of them (sub-step 0), and in 64-byte row pieces of
+    // one step each, they set the time of a step: 512 x 17408 x 5120 took 121
+    // us, 109 with the codes behind the A DMAs, 102 with them in 128-byte
+    // pieces too (85 without any code traffic); 4096 x 17408 x 5120, where the
+    // clock falls, 629, 607, 600.
+    static constexpr int B_DMA_EVERY = MFMAS / 8;
+    // Vector-memory operations issued after the last scale load of an
+    // iteration's last step: the MT A DMAs of sub-step 2.
+    static constexpr int VM_AFTER_SCALE = MT;
     // Sub-step of the 4 code reads of B(kt+2): the last with at least 4
     // MFMAs after them before the next step's first wait (that DMA is
     // complete from sub-step 1's wait on).
@@ -79,8 +86,8 @@ struct Geo {
 };
 constexpr int kBMMax = Geo<8>::BM;
 
-// Chunk swizzles: A rows hold 8 chunks of 16 B (slot = chunk ^ ga(row)), B
-// rows 4 chunks (slot = chunk ^ gb(row)).  For any 16 consecutive rows read
+// Chunk swizzles: A and B rows hold 8 chunks of 16 B (slot = chunk ^ ga(row));
+// gb does the same for rows of 4 chunks.  For any 16 consecutive rows read
 // at one chunk index both keep the 16-byte slots on distinct LDS banks.
 __device__ __forceinline__ int ga(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 __device__ __forceinline__ int gb(int r) { return ((r >> 1) ^ (r >> 3)) & 3; }
@@ -238,40 +245,40 @@ template <int MT>
 struct Ctx {
     i32x4 dx, dw, ds;
     uint32_t aoff[MT];  // A DMA lane offsets (k = 0)
-    uint32_t boff[4];   // B DMA lane offsets (k = 0)
+    uint32_t boff[8];   // B DMA lane offsets (k = 0)
     uint32_t soff[NT];  // scale row offsets
     uint32_t ard[4];    // A fragment read address per sub-step, stage 0
-    uint32_t brd[2];    // B read address per chunk pair, slot 0
+    uint32_t brd[2][2];  // B read address per step parity and chunk pair, slot 0
     uint32_t m0a, m0b;  // this wave's DMA LDS bases, stage / slot 0
     int scol;           // bytes per 128-K scale block in a scale row (4, or 0 for per-row scales)
 };
 
-// LDS positions of one step; the mod-3 rings are rotated at run time.
+// LDS positions of one step; the A ring is rotated at run time (the two B
+// slots alternate every two steps, which T fixes).
 struct Ring {
     uint32_t ar, an, aw;  // A stages kt%3 (read), (kt+1)%3 (next), (kt+2)%3 (DMA)
-    uint32_t bw, br;      // B slots kt%3 (DMA), (kt+2)%3 (read)
     __device__ __forceinline__ void advance() {
         const uint32_t t = ar;
         ar = an;
         an = aw;
         aw = t;
-        br = bw;
-        bw = bw == 2 * B_SLOT ? 0u : bw + B_SLOT;
     }
 };
 
 // Step kt, T = kt % 4.
 //   A: read stage kt%3; after the mid-step barrier DMA A(kt+2) into stage
 //      (kt+2)%3; in sub-step 3 read step kt+1's first fragments.
-//   B: DMA B(kt+3) into slot kt%3; dequantize B(kt+1) from braw[(kt+1)&1];
-//      in sub-step 3 (2 for 128-row tiles) read B(kt+2) from slot (kt+2)%3 into braw[kt&1].
+//   B: dequantize B(kt+1) from braw[(kt+1)&1]; in sub-step 3 (2 for 128-row
+//      tiles) read B(kt+2) from slot (kt/2+1)%2 into braw[kt&1]; in sub-step 3
+//      of an even step DMA B(kt+4) and B(kt+5) into slot (kt/2)%2, whose codes
+//      steps kt-2 and kt-1 read.
 //   Scales: odd steps load block (kt+3)/2 into bsc[block&1]; step kt
 //      dequantizes with block (kt+1)/2.
 // Per sub-step, slot m (one MFMA, then DQ dequant instructions) also carries:
 //   m < MT: the next sub-step's A fragment m (LDS read);
-//   sub-step 0: the 4 B DMAs (Geo::b_dma_at), and on odd steps the 2 scale
-//     loads in slots MT + 1, MT + 3;
+//   sub-step 0: on odd steps the 2 scale loads in slots MT + 1, MT + 3;
 //   sub-step 2, m >= MT: A DMA m - MT;
+//   sub-step 3 of even steps, every B_DMA_EVERY slots: the 8 B DMAs;
 //   sub-step BRAW_SUB, MT <= m < MT + 4: the 4 code reads of B(kt+2).
 template <int MT, int T>
 __device__ __forceinline__ void kstep(State<MT>& st, const Ctx<MT>& c, const Ring& rg, int kt) {
@@ -284,15 +291,16 @@ __device__ __forceinline__ void kstep(State<MT>& st, const Ctx<MT>& c, const Rin
     constexpr int NS = SLOAD ? 2 : 0;
     constexpr bool PREV_SLOAD = !(T & 1);
     constexpr int SB_PREV = ((T + 2) / 2) & 1;
-    const int kB = (kt + 3) * BK;
+    constexpr bool BLOAD = !(T & 1);
+    constexpr int SLOT_W = (T >> 1) & 1, SLOT_R = SLOT_W ^ 1;
+    const int kB = (kt + 4) * BK;
     const int kA = (kt + 2) * BK * 2;
     const int sS = ((kt + 3) >> 1) * c.scol;
     uint32_t ard[4];
 #pragma unroll
     for (int q = 1; q < 4; ++q) ard[q] = c.ard[q] + rg.ar;
     ard[0] = c.ard[0] + rg.an;
-    const uint32_t brd0 = c.brd[0] + rg.br, brd1 = c.brd[1] + rg.br;
-    const uint32_t m0b = c.m0b + rg.bw, m0a = c.m0a + rg.aw;
+    const uint32_t m0b = c.m0b + SLOT_W * B_SLOT, m0a = c.m0a + rg.aw;
 
     [&]<int... S>(std::integer_sequence<int, S...>) __attribute__((always_inline)) {
         ([&]() __attribute__((always_inline)) {
@@ -315,27 +323,28 @@ __device__ __forceinline__ void kstep(State<MT>& st, const Ctx<MT>& c, const Rin
                         else
                             ds_read<m * 4096>(st.af[0][m], ard[0]);
                     }
-                    if constexpr (s == 0 && Gm::b_dma_at(m)) {
-                        constexpr int g = Gm::b_dma_index(m);
-                        dma16(m0b + g * 1024, c.boff[g], c.dw, kB);
-                    }
                     if constexpr (SLOAD && s == 0 && (m == MT + 1 || m == MT + 3))
                         buf_load1(st.bsc[SB_LD][(m - MT - 1) >> 1], c.soff[(m - MT - 1) >> 1], c.ds, sS);
                     if constexpr (s == 2 && m >= MT)
                         dma16(m0a + (m - MT) * 1024, c.aoff[m - MT], c.dx, kA);
                     if constexpr (s == Gm::BRAW_SUB && m >= MT && m < MT + 4) {
                         constexpr int jj = (m - MT) >> 1, cp = (m - MT) & 1;
-                        ds_read<jj * 2048>(st.braw[RB_RD][jj][cp], cp ? brd1 : brd0);
+                        ds_read<SLOT_R * B_SLOT + jj * 4096>(st.braw[RB_RD][jj][cp], c.brd[T & 1][cp]);
+                    }
+                    if constexpr (BLOAD && s == 3 && m % Gm::B_DMA_EVERY == 0) {
+                        constexpr int g = m / Gm::B_DMA_EVERY;
+                        dma16(m0b + g * 1024, c.boff[g], c.dw, kB);
                     }
                 }(), ...);
             }(std::make_integer_sequence<int, Gm::MFMAS>{});
             if constexpr (s == 1) {
-                // A(kt+1), the previous step's last DMA, has landed (issued
-                // after it: this step's 4 B DMA and NS scale loads).
+                // A(kt+1) has landed, and on even steps B(kt+2) and B(kt+3)
+                // (issued after A(kt+1): an even previous step's 8 B DMA and
+                // this step's NS scale loads).
                 if constexpr (PREV_SLOAD)
-                    wait_vm2<4 + NS>(st.bsc[SB_PREV]);
+                    wait_vm2<0>(st.bsc[SB_PREV]);
                 else
-                    wait_vm<4 + NS>();
+                    wait_vm<8 + NS>();
                 barrier();
             }
         }(), ...);
@@ -452,12 +461,12 @@ __device__ __forceinline__ void setup(Ctx<MT>& c, const Unit& w, const uint16_t*
         c.aoff[ii] = m < M ? (uint32_t)((int64_t)m * K * 2 + ch * 16) : kBufferOob;
     }
     c.m0a = __builtin_amdgcn_readfirstlane(lds0 + wave * MT * 1024);
-    // B DMA instruction gi fills rows 16gi..16gi+15 of a slot: lane -> row
-    // 16gi + lane/4, LDS slot lane%4 <- chunk slot ^ gb(row).
+    // B DMA instruction gi fills rows 8gi..8gi+7 of a slot: lane -> row
+    // 8gi + lane/8, LDS slot lane%8 <- chunk slot ^ ga(row).
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) {
-        const int rr = 16 * gi + (lane >> 2);
-        const int ch = (lane & 3) ^ gb(rr);
+    for (int gi = 0; gi < 8; ++gi) {
+        const int rr = 8 * gi + (lane >> 3);
+        const int ch = (lane & 7) ^ ga(rr);
         const int64_t n = weight_row<SWIGLU>(w.ntile, wave, rr, N);
         c.boff[gi] = n >= 0 ? (uint32_t)(n * K + ch * 16) : kBufferOob;
     }
@@ -473,21 +482,19 @@ __device__ __forceinline__ void setup(Ctx<MT>& c, const Unit& w, const uint16_t*
         c.ard[s] = lds0 + l32 * 128 + 16 * (ch ^ ga(l32));
     }
 #pragma unroll
-    for (int cp = 0; cp < 2; ++cp)
-        c.brd[cp] = lds0 + A_BYTES + wave * B_WAVE + l32 * 64 + 16 * ((2 * cp + h) ^ gb(l32));
+    for (int q = 0; q < 4; ++q)
+        c.brd[q >> 1][q & 1] = lds0 + A_BYTES + wave * B_WAVE + l32 * 128 + 16 * ((2 * q + h) ^ ga(l32));
 }
 
 // Prologue loads of a unit, in the order the first step needs them: A(0)
-// into stage 0, B(0) and B(1) into slots 0 and 1, scale blocks 0 and 1, then
-// A(1) into stage 1 and B(2) into slot 2 (the last MT + 4 loads).
+// into stage 0, B(0) and B(1) into slot 0, scale blocks 0 and 1, then A(1)
+// into stage 1, B(2) and B(3) into slot 1 (the last MT + 8 loads).
 template <int MT>
 __device__ __forceinline__ void issue_prologue(State<MT>& st, const Ctx<MT>& c) {
 #pragma unroll
     for (int ii = 0; ii < MT; ++ii) dma16(c.m0a + ii * 1024, c.aoff[ii], c.dx, 0);
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int gi = 0; gi < 4; ++gi) dma16(c.m0b + p * B_SLOT + gi * 1024, c.boff[gi], c.dw, p * BK);
+    for (int gi = 0; gi < 8; ++gi) dma16(c.m0b + gi * 1024, c.boff[gi], c.dw, 0);
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         buf_load1(st.bsc[0][j], c.soff[j], c.ds, 0);
@@ -496,27 +503,26 @@ __device__ __forceinline__ void issue_prologue(State<MT>& st, const Ctx<MT>& c) 
 #pragma unroll
     for (int ii = 0; ii < MT; ++ii) dma16(c.m0a + Geo<MT>::A_STAGE + ii * 1024, c.aoff[ii], c.dx, BK * 2);
 #pragma unroll
-    for (int gi = 0; gi < 4; ++gi) dma16(c.m0b + 2 * B_SLOT + gi * 1024, c.boff[gi], c.dw, 2 * BK);
+    for (int gi = 0; gi < 8; ++gi) dma16(c.m0b + B_SLOT + gi * 1024, c.boff[gi], c.dw, 2 * BK);
 }
 
 // The rest of the prologue once A(0), B(0), B(1) and the scales have landed
-// (at most the MT + 4 loads of A(1) and B(2), or later stores, still in
+// (at most the MT + 8 loads of A(1), B(2) and B(3), or later stores, still in
 // flight): B(0) dequantized, B(1) codes and step 0's first A fragments read;
 // the accumulators cleared.  Step 0 first touches A(1) and B(2) after its
-// mid-step wait, which leaves only that step's own loads in flight, so
-// those two need no wait here; the kernel starts its first step about 1 us
-// earlier than with everything waited for (M = 512: 4.3 against 5.5 us
-// from launch to the first MFMA).
+// mid-step wait, so those need no wait here; the kernel starts its first step
+// about 1 us earlier than with everything waited for (M = 512: 4.3 against
+// 5.5 us from launch to the first MFMA).
 template <int MT>
 __device__ __forceinline__ void finish_prologue(State<MT>& st, const Ctx<MT>& c) {
-    wait_vm4<MT + 4>(st.bsc[0], st.bsc[1]);
+    wait_vm4<MT + 8>(st.bsc[0], st.bsc[1]);
     barrier();
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
         for (int cp = 0; cp < 2; ++cp) {
-            ds_read<0>(st.braw[0][j][cp], c.brd[cp] + j * 2048);
-            ds_read<B_SLOT>(st.braw[1][j][cp], c.brd[cp] + j * 2048);
+            ds_read<0>(st.braw[0][j][cp], c.brd[0][cp] + j * 4096);
+            ds_read<0>(st.braw[1][j][cp], c.brd[1][cp] + j * 4096);
         }
     wait_lgkm_braw<0>(st.braw);
     [&]<int... K2>(std::integer_sequence<int, K2...>) __attribute__((always_inline)) {
@@ -524,7 +530,12 @@ __device__ __forceinline__ void finish_prologue(State<MT>& st, const Ctx<MT>& c)
     }(std::make_integer_sequence<int, 128>{});
 #pragma unroll
     for (int i = 0; i < MT; ++i) ds_read<0>(st.af[0][i], c.ard[0] + i * 4096);
-    const u32x4 zero{0u, 0u, 0u, 0u};
+    // The MFMAs are inline asm, so the compiler does not keep the wait states
+    // between a VALU write of their operands and their read: write the zeros,
+    // then wait.  (Without it the first accumulator was cleared from stale
+    // registers wherever the allocation put the write right before it.)
+    u32x4 zero{0u, 0u, 0u, 0u};
+    asm volatile("s_nop 7" : "+v"(zero));
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -566,7 +577,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_kernel(const uint16_t* __rest
         // ---- K loop, 4 steps per iteration; only LDS DMA stays in flight
         // across the back edge.
         const int KT = cur.klen / BK;
-        Ring rg{0u, (uint32_t)Gm::A_STAGE, (uint32_t)(2 * Gm::A_STAGE), 0u, (uint32_t)(2 * B_SLOT)};
+        Ring rg{0u, (uint32_t)Gm::A_STAGE, (uint32_t)(2 * Gm::A_STAGE)};
         for (int kt = 0; kt < KT; kt += 4) {
             kstep<MT, 0>(st, c, rg, kt);
             rg.advance();
@@ -577,8 +588,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_kernel(const uint16_t* __rest
             kstep<MT, 3>(st, c, rg, kt + 3);
             rg.advance();
             // step kt+3 read step kt+4's fragments and B(kt+5) (LDS) and loaded
-            // scale block (kt+6)/2 into bsc[1], followed by VM_AFTER_SCALE DMA
-            // (10 for 256-row tiles, 4 for 128).
+            // scale block (kt+6)/2 into bsc[1], followed by VM_AFTER_SCALE DMA.
             wait_lgkm_ab<0>(st.af[0], st.braw[1]);
             wait_vm2<Gm::VM_AFTER_SCALE>(st.bsc[1]);
         }
