@@ -358,9 +358,14 @@ class LinearEngine:
     def linear(self, x, name, return_path=False):
         """`Engine::linear(x, name)` on one rank (src/engine.cpp:196-242): the
         branch, then the `name.bias` add; the cross-rank reduce is not run."""
+        # Small calls are bound by this function and the launch, not the kernel
+        # (two rows of 4096 x 4096: 11.5 us a call, 6 of them the kernel): no
+        # tensor operation that would change nothing, no query whose answer is 0.
+        flat = x.dim() == 2
         rows = x.numel() // x.size(-1)
-        x2 = x.reshape(rows, x.size(-1)).contiguous()
-        stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
+        x2 = x if flat and x.is_contiguous() else x.reshape(rows, x.size(-1)).contiguous()
+        device = x.device
+        stream = torch.cuda.current_stream(device).cuda_stream
         opt = self.options
         if name in self.mixed_projections:
             recs = [self._record(c) for c in self.mixed_projections[name]]
@@ -379,17 +384,17 @@ class LinearEngine:
             out = y.reshape(*x.shape[:-1], total)
             return (out, None) if return_path else out
         rec = self._record(name)
-        y = torch.empty((rows, rec.N), dtype=torch.bfloat16, device=x.device)
-        need = lib().fp8lin_engine_linear_workspace_bytes(ctypes.byref(opt), ctypes.byref(rec), rows)
-        ws = self._ws(need, x.device)
+        y = torch.empty((rows, rec.N), dtype=torch.bfloat16, device=device)
+        # optimized calls of up to 8 rows need no workspace on any branch
+        need = 0 if rows <= 8 and opt.optimized else lib().fp8lin_engine_linear_workspace_bytes(
+            ctypes.byref(opt), ctypes.byref(rec), rows)
+        ws = self._ws(need, device)
         path = ctypes.c_int(0)
-        end = self._profile_begin(name, x.device)
+        end = self._profile_begin(name, device)
         check(lib().fp8lin_engine_linear(
-            ctypes.byref(opt), ctypes.byref(rec), ctypes.c_void_p(x2.data_ptr()), rows,
-            ctypes.c_void_p(y.data_ptr()), rec.N,
-            ctypes.c_void_p(ws.data_ptr()) if ws is not None else None, need,
-            ctypes.byref(path), stream))
-        self._profile_end(end, x.device)
+            ctypes.byref(opt), ctypes.byref(rec), x2.data_ptr(), rows, y.data_ptr(), rec.N,
+            ws.data_ptr() if ws is not None else None, need, ctypes.byref(path), stream))
+        self._profile_end(end, device)
         self._count(path.value)
-        out = y.reshape(*x.shape[:-1], rec.N)
+        out = y if flat else y.reshape(*x.shape[:-1], rec.N)
         return (out, path.value) if return_path else out
