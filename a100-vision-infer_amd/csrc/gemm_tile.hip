@@ -30,10 +30,14 @@ constexpr Tile tile(int slots, float tau, float tau1) {
 }
 
 // BF16 weights, M x N x K in us (torch's mm, hipBLASLt, beside it): 1036 x 3456
-// x 1152 13.4 (24.5), 1036 x 4304 x 1152 19.7 (21.1), 1036 x 1152 x 4304 28
+// x 1152 13.4 (24.5), 1036 x 4304 x 1152 18.0 (21.1), 1036 x 1152 x 4304 28
 // (31), 40 x 7168 x 5120 19.9 (22.3), 300 x 5120 x 5120 30.5 (35.8), 4096 x
-// 8192 x 8192 456 (355: the library's large tile is the better one).  The
+// 8192 x 8192 474 (355: the library's large tile is the better one).  The
 // 256x256-only kernel this replaced took 47, 46, 571 (K % 64 != 0), 159.
+// 192x128 and 256x160 stand where 128x128 would need another round of
+// workgroups or 256x256 leave CUs idle: 1036 x 4304 x 1152 18.0 (19.7 without
+// them), 1036 x 5120 x 5120 60 (76), 2048 x 4304 x 1152 28.5 (34.2), 2048 x
+// 5120 x 5120 103 (124), 4096 x 5120 x 5120 207 (236).
 // E4M3FN codes, M x N x K in us (before: the persistent GEMM or, at K % 256,
 // the general template): 93 x 17408 x 5120 40 (47), 93 x 5120 x 8704 25.7
 // (34.8), 200 x 7168 x 5120 33.6 (40.1), 512 x 2048 x 2048 11.9 (26.3), 320 x
@@ -53,6 +57,8 @@ const Tile kBf16[] = {
     tile<Cfg<false, 128, 64, 2, 1, 4, 128, 3, false>, false>(1, 0.68f, 0.68f),
     tile<Cfg<false, 128, 128, 2, 2, 2, 64, 4, true>, false>(1, 0.98f, 0.98f),
     tile<Cfg<false, 128, 128, 2, 2, 1, 64, 2, false>, false>(2, 1.80f, 1.15f),
+    tile<Cfg<false, 192, 128, 2, 2, 2, 64, 4, true>, false>(1, 1.33f, 1.33f),
+    tile<Cfg<false, 256, 160, 4, 1, 1, 64, 3, true>, false>(1, 2.35f, 2.35f),
     tile<Cfg<false, 256, 256, 2, 4, 1, 64, 2, false>, false>(1, 3.10f, 3.10f),
 };
 const Tile kFp8[] = {

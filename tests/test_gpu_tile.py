@@ -17,11 +17,12 @@ def sample(m):
     return np.arange(m) if m <= 64 else np.unique(np.r_[0, 31, 32, 63, 64, 127, 128, m // 2, m - 2, m - 1].clip(0, m - 1))
 
 
-# One row per tile (32x32, 64x32, 64x64, 128x64, 128x128 with K over two
-# waves, 128x128 at two per CU, 256x256), then a shape with whole steps.
-@pytest.mark.parametrize("m,n,k", [(9, 261, 40), (515, 257, 1160), (33, 4100, 136), (9, 8200, 200), (65, 8195, 136),
-                                   (65, 17412, 200), (2050, 4100, 72), (2050, 2052, 136), (2050, 17412, 40),
-                                   (256, 2048, 512)])
+# One row per tile (32x32, 64x32, 64x64, 128x64, 128x128 with K over two waves
+# and at two per CU, 192x128, 256x160, 256x256), then longer K and whole steps.
+@pytest.mark.parametrize("m,n,k", [(9, 261, 40), (33, 4100, 136), (9, 8200, 200), (65, 8195, 136), (65, 17412, 200),
+                                   (2050, 17412, 40), (129, 17412, 136), (2050, 4100, 136), (2050, 6658, 136),
+                                   (515, 257, 1160), (1036, 4307, 1160), (2050, 4300, 1160), (2050, 2052, 136),
+                                   (129, 17412, 40), (256, 2048, 512)])
 def test_bf16_tile(fp8lin, gpu, oracle, m, n, k):
     """BF16 weights with a bias through the engine: the rows of the oracle's
     product, the bias added to the rounded outputs, and no row touched by
