@@ -117,11 +117,12 @@ int fp8lin_linear_ld(const uint16_t* x, const uint8_t* codes, const float* scale
  * projections at M = 512, or the 5120-row down projection at M = 65..128),
  * or leave a last round on at most half of them, those tiles are cut into
  * K ranges and a second launch adds their FP32 sums in order and rounds
- * once.  Within the parity bar of fp8lin_linear (only the FP32 summation
- * order of the split tiles differs); every other call is fp8lin_linear bit
- * for bit.  The workspace is what fp8lin_linear_workspace_bytes reports for
- * (M, N, K) (0: none needed; 256 KiB per split tile and K range), 16-byte
- * aligned, any content.  Replaces the same `fp8_linear` as fp8lin_linear;
+ * once.  Where smaller tiles, whole or in K ranges, are estimated faster
+ * than that, they run instead.  Within the parity bar of fp8lin_linear (only
+ * the FP32 summation order differs); up to 8 rows every call is
+ * fp8lin_linear bit for bit.  The workspace is what
+ * fp8lin_linear_workspace_bytes reports for (M, N, K) (0: none needed),
+ * 16-byte aligned, any content.  Replaces the same `fp8_linear` as fp8lin_linear;
  * the reference allocates such partials inside its own operator
  * (src/fp8_tensor.cu:65), here the caller passes them.
  */
@@ -144,10 +145,10 @@ int fp8lin_linear_swiglu(const uint16_t* x, const uint8_t* codes, const float* s
 
 /* The same with a workspace, which lets the prefill GEMM (M > 8) split K
  * where whole tiles would leave CUs idle: when the 256x256 tiles number
- * fewer than half the CUs, or leave a last round on at most a quarter of
+ * fewer than half the CUs, or leave a last round on at most half of
  * them (M = 1024 and M = 4096 at N = 17408, K = 5120), those tiles are cut
  * into K ranges whose FP32 sums a second launch adds in order before the
- * SwiGLU rounding points.  Within the parity bar of the unsplit call (only
+ * SwiGLU rounding points, or to run smaller tiles.  Within the parity bar of the unsplit call (only
  * the FP32 summation order of the split tiles differs).  The workspace is
  * what fp8lin_linear_swiglu_workspace_bytes reports (0: none needed), 16-byte
  * aligned.  Same replacement as fp8lin_linear_swiglu.
