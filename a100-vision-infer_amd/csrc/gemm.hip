@@ -75,8 +75,9 @@ size_t plan_bytes(const gemm_fp8::Plan& p) {
 // padding.  Above that the 256-row tile stays: measured on MI355X, a 128-row
 // tile costs 0.62 (whole chip) to 0.77 (one partial round) of a 256-row tile
 // (its K loop issues 4 dequant VALU per MFMA instead of 2, with the same
-// per-step waits), so two of them cost more than the one they replace.
-// Both heights give each output the same FP32 sum over a K range.
+// per-step waits), so two of them cost more than the one they replace; 192-row
+// tiles stand where they pay (route).  Every height gives each output the same
+// FP32 sum over a K range.
 gemm_fp8::Plan make_plan(int M, int N, int K, bool swiglu, int G, bool split) {
     return plan_for(M <= 128 ? 128 : 256, M, N, K, swiglu, G, split);
 }
@@ -103,8 +104,9 @@ hipError_t run_fp8_mt(const uint16_t* x, const uint8_t* w, const float* scales, 
 template <bool SWIGLU>
 hipError_t run_fp8(const uint16_t* x, const uint8_t* w, const float* scales, int S, uint16_t* y, int64_t ldy,
                    int M, int N, int K, const gemm_fp8::Plan& plan, int G, float* part, hipStream_t stream) {
-    return plan.bm == 128 ? run_fp8_mt<4, SWIGLU>(x, w, scales, S, y, ldy, M, N, K, plan, G, part, stream)
-                          : run_fp8_mt<8, SWIGLU>(x, w, scales, S, y, ldy, M, N, K, plan, G, part, stream);
+    if (plan.bm == 128) return run_fp8_mt<4, SWIGLU>(x, w, scales, S, y, ldy, M, N, K, plan, G, part, stream);
+    if (plan.bm == 192) return run_fp8_mt<6, SWIGLU>(x, w, scales, S, y, ldy, M, N, K, plan, G, part, stream);
+    return run_fp8_mt<8, SWIGLU>(x, w, scales, S, y, ldy, M, N, K, plan, G, part, stream);
 }
 
 // Shapes and alignments the FP8 kernel takes.
@@ -198,13 +200,20 @@ int compute_units() {
 namespace {
 
 // Estimated us of the persistent FP8 GEMM under plan p, from its measured
-// times: 4.8 us per 256 K and round of 256-row tiles (6.1 where whole rounds
-// fill the chip and its clock falls), 3.8 of 128-row tiles, and for a split
-// the partials' round trip and the second launch.
+// times: us per 256 K of a round of tiles, which grows with the share of the
+// CUs that run one (256-row tiles 4.3 at 0.53 of them, 5.0 at 0.80, 5.8 at
+// 0.98; 192-row tiles 3.7 at 0.66, 4.1 at 0.80, 4.8 at 0.98; whole rounds 6.1
+// and 5.0; 128-row tiles 3.8), and for a split the partials' round trip and
+// the second launch.
 float estimate(const gemm_fp8::Plan& p, int K, int G) {
-    const int chunks = K / 256;
+    const int chunks = K / 256, rounds = p.full / G;
+    const float share = (float)(p.full - rounds * G) / (float)G;
+    const float round = p.bm == 128 ? 3.8f : p.bm == 192 ? 5.0f : 6.1f;
+    const float last = p.bm == 128   ? 3.8f
+                       : p.bm == 192 ? 3.7f + 3.3f * std::max(0.0f, share - 0.66f)
+                                     : 4.3f + 3.2f * std::max(0.0f, share - 0.53f);
+    float us = 5.0f + (float)chunks * ((float)rounds * round + (share > 0.0f ? last : 0.0f));
     const float c = p.bm == 128 ? 3.8f : p.full >= G ? 6.1f : 4.8f;
-    float us = 5.0f + c * (float)(chunks * ((p.full + G - 1) / G));
     if (p.rtiles > 0)
         us += c * (float)((chunks + p.splits - 1) / p.splits) + 4.0f +
               8.0e-6f / 5.2f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
@@ -227,9 +236,17 @@ struct Route {
 Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, int K, bool swiglu, bool any, size_t have) {
     Route r{fp8_kernel_ok(x, w, S, ldy, M, N, K), false, {}, {}};
     const int G = compute_units();
+    // 192-row tiles, unsplit, where their round is the cheaper one: 256-row
+    // tiles that fill half the CUs to two thirds, or are half padding.  M x N x
+    // K without a workspace, 256-row tiles and 192: 512 x 17408 x 5120 91.6 and
+    // 87.6 us, 576 x 17408 x 5120 105.3 and 90.0, 300 x 17408 x 5120 87.9 and
+    // 72.4, 960 x 10240 x 5120 94.6 and 86.7, 1152 x 8704 x 5120 97.5 and 88.8.
+    // The required workspace stays the 256-row plan's.
     auto fitting = [&](bool sw) {
-        const gemm_fp8::Plan p = make_plan(M, N, K, sw, G, any);
-        return plan_bytes(p) <= have ? p : make_plan(M, N, K, sw, G, false);
+        gemm_fp8::Plan p = make_plan(M, N, K, sw, G, any);
+        if (plan_bytes(p) > have) p = make_plan(M, N, K, sw, G, false);
+        const gemm_fp8::Plan low = plan_for(192, M, N, K, sw, G, false);
+        return p.bm == 256 && estimate(low, K, G) < 0.99f * estimate(p, K, G) ? low : p;
     };
     if (r.gemm) r.plan = fitting(swiglu);
     if (tile_supported(x, w, true, S, M, N, K) && (!r.gemm || any)) {

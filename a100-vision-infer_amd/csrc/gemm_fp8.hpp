@@ -55,17 +55,21 @@ constexpr int B_WAVE = 2 * B_SLOT;
 // tile described above; MT = 4 (128 rows) serves launches of M <= 128 rows,
 // where a 256-row tile is at least half padding: the same K loop with half
 // the MFMAs per sub-step, so each code's dequantization (still once per
-// workgroup) costs 4 VALU per MFMA instead of 2.
+// workgroup) costs 4 VALU per MFMA instead of 2.  MT = 6 (192 rows) serves
+// launches whose 256-row tiles leave CUs idle where 192-row tiles still fit
+// one round of workgroups (gemm.hip).
 template <int MT>
 struct Geo {
-    static_assert(MT == 4 || MT == 8, "tile heights of 128 or 256 rows");
+    static_assert(MT == 4 || MT == 6 || MT == 8, "tile heights of 128, 192 or 256 rows");
     static constexpr int BM = 32 * MT;
     static constexpr int A_STAGE = BM * 128;  // BM rows x 64 BF16
     static constexpr int A_BYTES = 3 * A_STAGE;
-    static constexpr int LDS_BYTES = A_BYTES + 4 * B_WAVE;  // 160 KiB (MT 8) or 112 KiB (MT 4)
+    static constexpr int LDS_BYTES = A_BYTES + 4 * B_WAVE;  // 160 KiB (MT 8), 136 KiB (MT 6) or 112 KiB (MT 4)
     static constexpr int SLOT_FLOATS = BM * BN;             // one split partial
     static constexpr int MFMAS = 2 * MT;                    // per sub-step
-    static constexpr int DQ = 16 / MT;                      // dequant instructions per MFMA
+    // First of the 128 dequant instructions of a step that follow its MFMA n
+    // (2 per MFMA for MT 8, 4 for MT 4, 2 or 3 for MT 6).
+    static constexpr int dq(int n) { return n * 32 / MFMAS; }
     // The 8 B DMAs of an even step are spread over its sub-step 3, after the
     // step's A DMAs.  Vector-memory operations retire in order, so the next
     // step's mid-step wait for those A DMAs also waits for all that was issued
@@ -169,6 +173,13 @@ __device__ __forceinline__ void wait_lgkm_a(u32x4 (&a)[8]) {
                  : "memory");
 }
 template <int N>
+__device__ __forceinline__ void wait_lgkm_a(u32x4 (&a)[6]) {
+    asm volatile("s_waitcnt lgkmcnt(%6)"
+                 : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5])
+                 : "i"(N)
+                 : "memory");
+}
+template <int N>
 __device__ __forceinline__ void wait_lgkm_a(u32x4 (&a)[4]) {
     asm volatile("s_waitcnt lgkmcnt(%4)" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]) : "i"(N) : "memory");
 }
@@ -177,6 +188,14 @@ __device__ __forceinline__ void wait_lgkm_ab(u32x4 (&a)[8], u32x4 (&b)[NT][2]) {
     asm volatile("s_waitcnt lgkmcnt(%12)"
                  : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),
                    "+v"(b[0][0]), "+v"(b[0][1]), "+v"(b[1][0]), "+v"(b[1][1])
+                 : "i"(N)
+                 : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_lgkm_ab(u32x4 (&a)[6], u32x4 (&b)[NT][2]) {
+    asm volatile("s_waitcnt lgkmcnt(%10)"
+                 : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(b[0][0]), "+v"(b[0][1]),
+                   "+v"(b[1][0]), "+v"(b[1][1])
                  : "i"(N)
                  : "memory");
 }
@@ -268,13 +287,13 @@ struct Ring {
 // Step kt, T = kt % 4.
 //   A: read stage kt%3; after the mid-step barrier DMA A(kt+2) into stage
 //      (kt+2)%3; in sub-step 3 read step kt+1's first fragments.
-//   B: dequantize B(kt+1) from braw[(kt+1)&1]; in sub-step 3 (2 for 128-row
+//   B: dequantize B(kt+1) from braw[(kt+1)&1]; in sub-step 3 (2 for lower
 //      tiles) read B(kt+2) from slot (kt/2+1)%2 into braw[kt&1]; in sub-step 3
 //      of an even step DMA B(kt+4) and B(kt+5) into slot (kt/2)%2, whose codes
 //      steps kt-2 and kt-1 read.
 //   Scales: odd steps load block (kt+3)/2 into bsc[block&1]; step kt
 //      dequantizes with block (kt+1)/2.
-// Per sub-step, slot m (one MFMA, then DQ dequant instructions) also carries:
+// Per sub-step, slot m (one MFMA, then its dequant instructions) also carries:
 //   m < MT: the next sub-step's A fragment m (LDS read);
 //   sub-step 0: on odd steps the 2 scale loads in slots MT + 1, MT + 3;
 //   sub-step 2, m >= MT: A DMA m - MT;
@@ -315,8 +334,8 @@ __device__ __forceinline__ void kstep(State<MT>& st, const Ctx<MT>& c, const Rin
                     constexpr int i = m >> 1, j = m & 1;
                     mfma(st.acc[i][j], st.af[s & 1][i], st.bf[BC][j][s]);
                     [&]<int... D>(std::integer_sequence<int, D...>) __attribute__((always_inline)) {
-                        (dequant_op<(s * Gm::MFMAS + m) * Gm::DQ + D, RB_DQ, BD>(st, st.bsc[SB_DQ]), ...);
-                    }(std::make_integer_sequence<int, Gm::DQ>{});
+                        (dequant_op<Gm::dq(s * Gm::MFMAS + m) + D, RB_DQ, BD>(st, st.bsc[SB_DQ]), ...);
+                    }(std::make_integer_sequence<int, Gm::dq(s * Gm::MFMAS + m + 1) - Gm::dq(s * Gm::MFMAS + m)>{});
                     if constexpr (m < MT) {
                         if constexpr (s < 3)
                             ds_read<m * 4096>(st.af[(s + 1) & 1][m], ard[s + 1]);
@@ -331,7 +350,7 @@ __device__ __forceinline__ void kstep(State<MT>& st, const Ctx<MT>& c, const Rin
                         constexpr int jj = (m - MT) >> 1, cp = (m - MT) & 1;
                         ds_read<SLOT_R * B_SLOT + jj * 4096>(st.braw[RB_RD][jj][cp], c.brd[T & 1][cp]);
                     }
-                    if constexpr (BLOAD && s == 3 && m % Gm::B_DMA_EVERY == 0) {
+                    if constexpr (BLOAD && s == 3 && m % Gm::B_DMA_EVERY == 0 && m / Gm::B_DMA_EVERY < 8) {
                         constexpr int g = m / Gm::B_DMA_EVERY;
                         dma16(m0b + g * 1024, c.boff[g], c.dw, kB);
                     }
@@ -373,7 +392,7 @@ constexpr int kGroupM = 8;
 constexpr int kMaxSplits = 8;
 
 struct Plan {
-    int bm;              // tile height: 256 or 128 rows of M
+    int bm;              // tile height: 256, 192 or 128 rows of M
     int mtiles, ntiles;  // tile grid (ntiles counts 256-row weight blocks, or 128 output pairs for SwiGLU)
     int full;            // whole tiles
     int fpad;            // full rounded up to a multiple of 8

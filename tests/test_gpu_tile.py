@@ -110,6 +110,35 @@ def test_fp8_tile_beside_persistent_gemm(fp8lin, gpu, oracle, m, n, k):
     assert torch.equal(bad[keep], split[keep]) and torch.isnan(bad[m // 2]).all()
 
 
+# 192-row tiles of the persistent GEMM (two or three rows of them in one round
+# where 256-row tiles fill half the chip to all of it): one row into a tile,
+# one short of it, whole, ragged columns, the fewest K steps that choose them.
+@pytest.mark.parametrize("m,n,k", [(385, 17408, 1024), (512, 17300, 512), (575, 21504, 768), (576, 20002, 1280),
+                                   (512, 17408, 5120), (129, 33000, 512), (192, 32770, 1024)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_192_row_tiles(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """Unsplit sums do not depend on the tile height: bit for bit the rows of
+    calls of at most 128 rows (128-row tiles), which meet the oracle; SwiGLU
+    likewise; a row of NaN stays in its row."""
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random(n if rows_scaled else (n, k // 128)) * .01 + .001).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    x[m // 2] = 0x7fc0  # NaN
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    y = fp8lin.fp8_linear(xd, cd, sd, split=False)
+    assert torch.isnan(y[m // 2]).all()
+    parts = [fp8lin.fp8_linear(xd[i:i + 128], cd, sd, split=False) for i in range(0, m - 64, 128)]
+    low = torch.cat(parts)
+    assert torch.equal(y[:low.size(0)].nan_to_num(1e30), low.nan_to_num(1e30))
+    rows = np.array([0, 191, m - 1])
+    rows = rows[(rows < m) & (rows != m // 2)]
+    cols = np.r_[0:64, n - 64:n]
+    assert_parity(bits(y)[rows][:, cols], oracle.linear(x[rows], codes[cols], scales[cols]), f"192-row tiles {m}x{n}x{k}")
+    pair = fp8lin.linear_swiglu(xd, cd, sd, split=False)
+    assert torch.equal(pair.nan_to_num(1e30), fp8lin.fused_swiglu(y).nan_to_num(1e30))
+
+
 @pytest.mark.parametrize("m", [1, 4, 27, 70, 300])
 @pytest.mark.parametrize("option", ["plain", "bias", "cached", "dequant", "profiled"])
 def test_engine_mlp_swiglu_forms(fp8lin, gpu, oracle, m, option):
