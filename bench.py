@@ -30,16 +30,16 @@ METRIC = "FP8 GEMV HBM GB/s (% peak) at M=1; prefill GEMM TFLOP/s (% MFMA peak)"
 GATE_UP_TRAFFIC_BYTES = 92_152_013
 # One M=4096 gate/up+SwiGLU prefill call (gemm_fp8_kernel<8, true> and its
 # tail_reduce_kernel), copy-calibrated FETCH_SIZE x2 + WRITE_SIZE, rotated.
-PREFILL_TRAFFIC_BYTES = 1_119_594_086
+PREFILL_TRAFFIC_BYTES = 1_119_044_894
 # MFMA busy fraction of the prefill kernel over its whole dispatch (M=4096
 # gate/up+SwiGLU), one --pmc pass: SQ_VALU_MFMA_BUSY_CYCLES summed over the
 # 1024 SIMDs, per SIMD, over the dispatch's cycles.  GRBM_GUI_ACTIVE comes back
 # summed over the 8 XCDs (8 x the dispatch's cycles at the shader clock), so
 # rocprofv3's own MfmaUtil formula reads 8x low on this part.  Re-measure when
 # the kernel changes.
-PREFILL_MFMA_BUSY = 0.730
+PREFILL_MFMA_BUSY = 0.723
 PREFILL_MFMA_BUSY_SOURCE = ("rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES GRBM_GUI_ACTIVE: 715.7e6 busy cycles "
-                            "/ 1024 SIMDs over GRBM_GUI_ACTIVE / 8 XCDs = 0.957e6 cycles (1.60 GHz)")
+                            "/ 1024 SIMDs over GRBM_GUI_ACTIVE / 8 XCDs = 0.967e6 cycles (1.60 GHz)")
 SHAPES = [("gate_up", 17408, 5120), ("down", 5120, 8704), ("qkv_gate", 7168, 5120)]
 
 
