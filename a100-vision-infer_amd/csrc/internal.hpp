@@ -85,13 +85,15 @@ hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t
                             int N, int K, hipStream_t stream);
 
 // FP8 prefill GEMM (gemm.hip), M > 8, with a workspace for K-split partials
-// (or null; may_split false: an entry point that takes none): where whole tiles leave CUs idle K is split and a second launch
-// adds the FP32 partials.  gemm_workspace_bytes() is what the plan needs (0
-// when nothing splits); gemm_split_bytes() is the persistent GEMM's own part
-// of it.  A smaller or unaligned workspace, unaligned x or w, or another
-// kernel's shape run unsplit.  The tiles add bias (or null) and set
-// *bias_added; the other kernels leave it to the caller.  When swiglu, N is the number of weight rows
-// (gate rows [0,N/2), up rows [N/2,N)) and y is [M, N/2].
+// (or null; may_split false: an entry point that takes none): where whole
+// tiles leave CUs idle K is split and a second launch adds the FP32 partials.
+// gemm_workspace_bytes() is what the plan needs (0 when nothing splits);
+// gemm_split_bytes() is the persistent GEMM's own part of it, of its 128- and
+// 256-row tiles.  A smaller or unaligned workspace, unaligned x or w, or
+// another kernel's shape run unsplit.  The tiles add bias (or null) and set
+// *bias_added; the other kernels leave it to the caller.  When swiglu, N is
+// the number of weight rows (gate rows [0,N/2), up rows [N/2,N)) and y is
+// [M, N/2].
 size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 // Whether the GEMM dispatch sends this FP8 call (9..32 rows) to the small-M
