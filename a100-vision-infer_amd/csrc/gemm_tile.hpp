@@ -260,13 +260,16 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
     constexpr int SETS = C::PIPE ? 2 : 1;
     u32x4 a[SETS][C::NT][2], b[SETS][C::MT][2], raw[C::NT];
     float scl[C::NT];
+    const int klim = K - 16 * h;
     auto fetch = [&](int set, uint32_t stage, int s, int t) __attribute__((always_inline)) {
         if constexpr (C::FP8) {
             const int kb = S == 1 ? 0 : min((((t0 + t) * C::BK) >> 7) - kb0, SB - 1);
+            // a chunk past K holds zero codes; its scale must be zero too (0 * inf)
+            const bool in_k = (t0 + t) * C::BK + 32 * s < klim;
 #pragma unroll
             for (int j = 0; j < C::NT; ++j) {
                 raw[j] = lds16(wrow + stage + j * 32 * C::WROW + 16 * swz<CHW>(l32, 2 * s + h));
-                scl[j] = srow[j * 32 * sstride + kb];
+                scl[j] = in_k ? srow[j * 32 * sstride + kb] : 0.0f;
             }
         } else {
 #pragma unroll

@@ -86,6 +86,28 @@ def test_fp8_tile(fp8lin, gpu, oracle, m, n, k, rows_scaled):
             assert torch.equal(fp8lin.linear_swiglu(xd, cd, sd, split=split), fp8lin.fused_swiglu(y))
 
 
+@pytest.mark.parametrize("m,n,k", FP8_TILES)
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_tile_infinite_scale(fp8lin, gpu, m, n, k, rows_scaled):
+    """K ends inside a step of every shape: the zeros past it add nothing also
+    where the scale they share with the last codes is infinite.  Positive codes
+    and activations, so those outputs are +inf; all others keep their bits."""
+    rng = np.random.default_rng(m + 3 * n + k)
+    codes = up(rng.integers(1, 127, (n, k), dtype=np.uint8), gpu)
+    scales = up((rng.random(n if rows_scaled else (n, (k + 127) // 128)) * .01 + .001).astype(np.float32), gpu)
+    x = up(rand_bf16(rng, (m, k)) & 0x7fff | 1, gpu)
+    cols = [0, n // 2, n - 1]
+    bad = scales.clone()
+    if rows_scaled:
+        bad[cols] = float("inf")
+    else:
+        bad[cols, -1] = float("inf")
+    for split in (False, True):
+        ref = fp8lin.fp8_linear(x, codes, scales, split=split)
+        ref[:, cols] = float("inf")
+        assert torch.equal(fp8lin.fp8_linear(x, codes, bad, split=split), ref)
+
+
 @pytest.mark.parametrize("m,n,k", [(70, 4096, 2048), (93, 5120, 3072), (129, 2048, 1024), (200, 1536, 4096),
                                    (320, 2048, 2048), (513, 1030, 1280), (65, 17408, 4096)])
 def test_fp8_tile_beside_persistent_gemm(fp8lin, gpu, oracle, m, n, k):
