@@ -139,13 +139,13 @@ bool linear_small_m(const uint16_t* x, const uint8_t* codes, int64_t S, int64_t 
     return M > 2 || K > 5120 || fp8lin::small_m_two_rows((int)N, (int)K);
 }
 
-// K-split partials of fp8_linear's prefill GEMM (M > 8) for output row stride
-// ldy: the engine branch's plan (few tiles, or a small last round, split K);
-// 0 where nothing splits.  Block scales are assumed: per-row scales take the
-// same plan.
-size_t linear_ws(int64_t M, int64_t N, int64_t K, int64_t ldy) {
-    if (M <= 8 || M >= kMaxDim || N <= 0 || N >= kMaxDim || K <= 0 || K >= kMaxDim) return 0;
-    return fp8lin::gemm_workspace_bytes((int)ceil_div(K, 128), ldy, (int)M, (int)N, (int)K, false);
+// K-split partials of fp8_linear's prefill GEMM (M > 8), or of its SwiGLU form,
+// for S scales a row: the engine branch's plan (few tiles, or a small last
+// round, split K); 0 where nothing splits.  The scale form decides: up to 64
+// rows of block scales run the small-M kernels, of row scales the GEMM.
+size_t linear_ws(int64_t M, int64_t N, int64_t K, int64_t S, bool swiglu) {
+    if (M <= 8 || M >= kMaxDim || N <= 0 || N >= kMaxDim || K <= 0 || K >= kMaxDim || (swiglu && N % 2)) return 0;
+    return fp8lin::gemm_workspace_bytes((int)S, swiglu ? N / 2 : N, (int)M, (int)N, (int)K, swiglu);
 }
 
 // The part of a GEMM workspace that a call is refused without: the persistent
@@ -531,7 +531,13 @@ int fp8lin_linear(const uint16_t* x, const uint8_t* codes, const float* scales, 
     return fp8lin_linear_ld(x, codes, scales, scale_cols, y, N, M, N, K, vector_gemv, stream);
 }
 
-size_t fp8lin_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) { return linear_ws(M, N, K, N); }
+size_t fp8lin_linear_workspace_bytes(int64_t M, int64_t N, int64_t K) {
+    return linear_ws(M, N, K, ceil_div(K, 128), false);
+}
+
+size_t fp8lin_linear_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t scale_cols) {
+    return linear_ws(M, N, K, scale_cols, false);
+}
 
 int fp8lin_linear_ws(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t scale_cols,
                      uint16_t* y, int64_t M, int64_t N, int64_t K, int vector_gemv, void* workspace,
@@ -581,8 +587,11 @@ int fp8lin_add_bias(uint16_t* y, int64_t ldy, const uint16_t* bias, int64_t rows
 }
 
 size_t fp8lin_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_t K) {
-    if (M <= 8 || N <= 0 || K <= 0 || N % 2 || M >= kMaxDim || N >= kMaxDim || K >= kMaxDim) return 0;
-    return fp8lin::gemm_workspace_bytes((int)ceil_div(K, 128), N / 2, (int)M, (int)N, (int)K, true);
+    return linear_ws(M, N, K, ceil_div(K, 128), true);
+}
+
+size_t fp8lin_linear_swiglu_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t scale_cols) {
+    return linear_ws(M, N, K, scale_cols, true);
 }
 
 int fp8lin_linear_swiglu_ws(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t scale_cols,

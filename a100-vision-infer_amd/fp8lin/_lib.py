@@ -44,6 +44,7 @@ EXPORTED = [
     "fp8lin_linear_candidates_static",
     "fp8lin_linear_swiglu_workspace_bytes", "fp8lin_linear_swiglu_ws",
     "fp8lin_linear_workspace_bytes", "fp8lin_linear_ws",
+    "fp8lin_linear_scaled_workspace_bytes", "fp8lin_linear_swiglu_scaled_workspace_bytes",
     "fp8lin_decode_chain_workspace_bytes", "fp8lin_decode_chain",
 ]
 
@@ -110,12 +111,14 @@ def lib():
         "fp8lin_linear": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i32, vp]),
         "fp8lin_linear_ld": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i64, i32, vp]),
         "fp8lin_linear_workspace_bytes": (sz, [i64, i64, i64]),
+        "fp8lin_linear_scaled_workspace_bytes": (sz, [i64, i64, i64, i64]),
         "fp8lin_decode_chain_workspace_bytes": (sz, [i32]),
         "fp8lin_decode_chain": (i32, [ctypes.POINTER(ChainLink), i32, vp, sz, vp]),
         "fp8lin_linear_ws": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i32, vp, sz, vp]),
         "fp8lin_linear_swiglu": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, vp]),
         "fp8lin_swiglu": (i32, [vp, vp, i64, i64, vp]),
         "fp8lin_linear_swiglu_workspace_bytes": (sz, [i64, i64, i64]),
+        "fp8lin_linear_swiglu_scaled_workspace_bytes": (sz, [i64, i64, i64, i64]),
         "fp8lin_linear_swiglu_ws": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, vp, sz, vp]),
         "fp8lin_add_bias": (i32, [vp, i64, vp, i64, i64, vp]),
         "fp8lin_linear_shared": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, vp]),

@@ -250,7 +250,7 @@ class LinearEngine:
                     ctypes.byref(self.options), ctypes.byref(rec), rows) in (PATH_FP8_GEMV, PATH_FP8_GEMM):
                 x = n.contiguous()
                 y = torch.empty((rows, rec.N // 2), dtype=torch.bfloat16, device=n.device)
-                need = lib().fp8lin_linear_swiglu_workspace_bytes(rows, rec.N, rec.K)
+                need = lib().fp8lin_linear_swiglu_scaled_workspace_bytes(rows, rec.N, rec.K, rec.scale_cols)
                 ws = self._ws(need, n.device)
                 check(lib().fp8lin_linear_swiglu_ws(
                     x.data_ptr(), rec.data, rec.scales, rec.scale_cols, y.data_ptr(), rows, rec.N, rec.K,

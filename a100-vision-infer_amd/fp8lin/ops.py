@@ -81,9 +81,9 @@ def fp8_linear(x, codes, scales, vector_gemv=False, split=True):
     """`at::Tensor fp8_linear(x, codes, scales, bool vector_gemv=false)` --
     src/optimized.cu:61-70.  split: give the prefill GEMM a workspace (allocated
     here, on the input's stream, as the reference allocates its operators'
-    partials, src/fp8_tensor.cu:65) so it may split K where whole tiles would
-    leave CUs idle (fp8lin_linear_ws); False runs every tile whole
-    (fp8lin_linear)."""
+    partials, src/fp8_tensor.cu:65) so it may split K, or take smaller tiles,
+    where whole tiles would leave CUs idle (fp8lin_linear_ws, as
+    LinearEngine.linear); False runs every tile whole (fp8lin_linear)."""
     _check_x(x, "FP8 linear expects CUDA BF16 [M,K]")
     _check_codes(codes, x)
     sc = _scale_cols(scales, codes.size(0), codes.size(1))
@@ -91,9 +91,9 @@ def fp8_linear(x, codes, scales, vector_gemv=False, split=True):
     if not (M > 0 and N > 0 and K > 0):
         _fail(ERR_SHAPE, "Empty GEMM")
     y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
-    need = lib().fp8lin_linear_workspace_bytes(M, N, K) if split else 0
-    if need:
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    if split:
+        need = lib().fp8lin_linear_scaled_workspace_bytes(M, N, K, sc)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
         check(lib().fp8lin_linear_ws(_ptr(x), _ptr(codes), _ptr(scales), sc, _ptr(y), M, N, K,
                                      int(bool(vector_gemv)), _ptr(ws), need, _stream(x)))
     else:
@@ -114,9 +114,9 @@ def linear_swiglu(x, codes, scales, split=True):
     if not (M > 0 and N > 0 and K > 0) or N % 2:
         _fail(ERR_SHAPE, "Invalid gate/up geometry")
     y = torch.empty((M, N // 2), dtype=torch.bfloat16, device=x.device)
-    need = lib().fp8lin_linear_swiglu_workspace_bytes(M, N, K) if split else 0
-    if need:
-        ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    if split:
+        need = lib().fp8lin_linear_swiglu_scaled_workspace_bytes(M, N, K, sc)
+        ws = torch.empty(need, dtype=torch.uint8, device=x.device) if need else None
         check(lib().fp8lin_linear_swiglu_ws(_ptr(x), _ptr(codes), _ptr(scales), sc, _ptr(y), M, N, K, _ptr(ws),
                                             need, _stream(x)))
     else:

@@ -121,12 +121,14 @@ int fp8lin_linear_ld(const uint16_t* x, const uint8_t* codes, const float* scale
  * than that, they run instead.  Within the parity bar of fp8lin_linear (only
  * the FP32 summation order differs); up to 8 rows every call is
  * fp8lin_linear bit for bit.  The workspace is what
- * fp8lin_linear_workspace_bytes reports for (M, N, K) (0: none needed),
- * 16-byte aligned, any content.  Replaces the same `fp8_linear` as fp8lin_linear;
+ * fp8lin_linear_workspace_bytes reports for block scales, and
+ * fp8lin_linear_scaled_workspace_bytes for scale_cols of either form (0: none
+ * needed), 16-byte aligned, any content.  Replaces the same `fp8_linear` as fp8lin_linear;
  * the reference allocates such partials inside its own operator
  * (src/fp8_tensor.cu:65), here the caller passes them.
  */
 size_t fp8lin_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t fp8lin_linear_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t scale_cols);
 int fp8lin_linear_ws(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t scale_cols,
                      uint16_t* y, int64_t M, int64_t N, int64_t K, int vector_gemv, void* workspace,
                      size_t workspace_bytes, fp8lin_stream_t stream);
@@ -150,10 +152,13 @@ int fp8lin_linear_swiglu(const uint16_t* x, const uint8_t* codes, const float* s
  * into K ranges whose FP32 sums a second launch adds in order before the
  * SwiGLU rounding points, or to run smaller tiles.  Within the parity bar of the unsplit call (only
  * the FP32 summation order of the split tiles differs).  The workspace is
- * what fp8lin_linear_swiglu_workspace_bytes reports (0: none needed), 16-byte
- * aligned.  Same replacement as fp8lin_linear_swiglu.
+ * what fp8lin_linear_swiglu_workspace_bytes reports for block scales, and
+ * fp8lin_linear_swiglu_scaled_workspace_bytes for scale_cols of either form
+ * (0: none needed), 16-byte aligned.  Same replacement as
+ * fp8lin_linear_swiglu.
  */
 size_t fp8lin_linear_swiglu_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t fp8lin_linear_swiglu_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t scale_cols);
 int fp8lin_linear_swiglu_ws(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t scale_cols,
                             uint16_t* y, int64_t M, int64_t N, int64_t K, void* workspace, size_t workspace_bytes,
                             fp8lin_stream_t stream);

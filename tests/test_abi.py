@@ -350,6 +350,23 @@ def test_linear_workspace_bytes_none(fp8lin, m, n, k):
     assert fp8lin.lib().fp8lin_linear_workspace_bytes(m, n, k) == 0
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 5120, 8704), (27, 8192, 5120), (32, 7168, 5120), (64, 5120, 8704),
+                                   (93, 5120, 8704), (512, 7168, 5120), (65, 4100, 4112), (4, 5120, 8704)])
+def test_linear_workspace_bytes_by_scale_form(fp8lin, m, n, k):
+    """The operators' queries answer for the weight's scale form, as the engine's
+    does: row scales run the GEMM where block scales run the small-M kernels."""
+    L = fp8lin.lib()
+    for cols in (1, -(-k // 128)):
+        w = fp8lin._lib.Weight(data=0x10000, scales=0x10000, scale_cols=cols, N=n, K=k)
+        opt = fp8lin.LinearOptions()
+        need = L.fp8lin_engine_linear_workspace_bytes(ctypes.byref(opt), ctypes.byref(w), m)
+        assert L.fp8lin_linear_scaled_workspace_bytes(m, n, k, cols) == need
+        assert L.fp8lin_linear_swiglu_scaled_workspace_bytes(m, n, k, cols) == need
+        assert (need > 0) == (m > 8 and (cols == 1 or m > 64))
+    assert L.fp8lin_linear_workspace_bytes(m, n, k) == need
+    assert L.fp8lin_linear_swiglu_workspace_bytes(m, n, k) == need
+
+
 def test_linear_ws_validation(fp8lin):
     """fp8lin_linear_ws checks its workspace before touching a device."""
     L = fp8lin.lib()

@@ -132,6 +132,29 @@ def test_fp8_tile_beside_persistent_gemm(fp8lin, gpu, oracle, m, n, k):
     assert torch.equal(bad[keep], split[keep]) and torch.isnan(bad[m // 2]).all()
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 5120, 8704), (27, 8192, 5120), (40, 2304, 7424), (64, 2304, 8192), (77, 4100, 2880),
+                                   (70, 32896, 6656), (200, 7168, 5120)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_engine_operator_and_fused_agree(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """The engine's projection, the operator and the fused gate/up of one weight
+    run one plan: the same bits, with row scales as with block scales (9..64
+    rows: the GEMM with row scales, the small-M kernels with block scales)."""
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random(n if rows_scaled else (n, (k + 127) // 128)) * .01 + .001).astype(np.float32)
+    x, c, s = up(rand_bf16(rng, (m, k)), gpu), up(codes, gpu), up(scales, gpu)
+    eng = fp8lin.LinearEngine()
+    eng.add("p.weight", c, s)
+    y = eng.linear(x, "p")
+    assert torch.equal(y, fp8lin.fp8_linear(x, c, s))
+    pair = fp8lin.fused_swiglu(y)
+    assert torch.equal(pair, fp8lin.linear_swiglu(x, c, s))
+    assert torch.equal(pair, eng._linear_swiglu(x, "p"))
+    cols = np.r_[0:32, n - 32:n]
+    rows = sample(m)
+    assert_parity(bits(y)[rows][:, cols], oracle.linear(bits(x)[rows], codes[cols], scales[cols]), f"{m}x{n}x{k}")
+
+
 # 192-row tiles of the persistent GEMM (two or three rows of them in one round
 # where 256-row tiles fill half the chip to all of it): one row into a tile,
 # one short of it, whole, ragged columns, the fewest K steps that choose them.
