@@ -107,6 +107,7 @@ Grid grid_of(const Tile& t, int M, int N, int64_t ldy, const uint16_t* y, const 
     g.ldp = ceil_div(N, 8) * 8 + 8;
     g.wide = (ldy % 8 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 ? 1 : 0) |
              (ldy % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 8 == 0 ? 4 : 0) |
+             (ldy % 2 == 0 && reinterpret_cast<uintptr_t>(y) % 4 == 0 ? 8 : 0) |
              (reinterpret_cast<uintptr_t>(bias) % 16 == 0 ? 2 : 0);
     // One round: spread the columns evenly over the CUs.
     g.per = t.bn;

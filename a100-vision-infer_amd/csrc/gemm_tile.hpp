@@ -67,6 +67,16 @@ struct Cfg {
     static_assert(X_STAGE % (1024 * WAVES) == 0 && W_STAGE % (1024 * WAVES) == 0, "equal DMA shares");
     static_assert(WK == 1 || BM * BN * 4 <= RING, "a partial tile fits the ring");
     static_assert(RING <= kLds, "LDS");
+    // Output rows off the 16-byte grid go through LDS (store_staged), in the part
+    // of the ring that each wave then has to itself; 4 is rows on 8 bytes, which
+    // the smaller tiles store as they are.  Lane's own rows and staged, us: 512 x
+    // 15137 x 1152 45.8 and 24.5, 2048 x 562 x 1152 14.8 and 12.2, 1036 x 625 x
+    // 1152 (FP8) 11.5 and 9.2; on 8 bytes 2048 x 9740 x 1152 66.5 and 58.9 (large
+    // tiles), 40 x 11004 x 1152 7.5 and 8.0 (64x64).
+    static constexpr bool STAGED = BM * BN >= 64 * 64;
+    static constexpr int DIRECT = BM * BN >= 128 * 128 ? 1 : 1 | 4;
+    static constexpr int STORE_BYTES = WK > 1 ? MT * NT * 4096 : 32 * (NT * 64 + 16);
+    static_assert(!STAGED || (STORE_BYTES >= 32 * (NT * 64 + 16) && WM * WN * STORE_BYTES <= RING), "32 rows of a wave's tile");
     // Ring and, for FP8, the rows' scales of the longest K range, padded to an
     // odd stride so that 32 rows at one block fall in distinct banks.
     static int lds_bytes(int S, int K, int splits) {
@@ -111,6 +121,42 @@ __device__ __forceinline__ void store8(uint16_t* dst, const uint32_t* o, int lef
                 if (r < left) dst[r] = (uint16_t)(o[r >> 1] >> (16 * (r & 1)));
         }
     }
+}
+
+// The first `left` of COLS columns and `rows` of 32 rows that the wave has just
+// put in LDS (rows of 2 COLS + 16 bytes) to dst, E outputs a lane, neighbouring
+// lanes on neighbouring outputs.  Where y's rows start off the 16-byte grid a
+// lane's own row in narrow stores touches a cache line per lane and store.  The
+// reads of a batch are all under way before its first store.
+template <int E, int COLS>
+__device__ __forceinline__ void store_staged(uint16_t* dst, int64_t ldy, const uint8_t* stage, int rows, int left) {
+    typedef uint16_t Out __attribute__((ext_vector_type(E)));
+    constexpr int LPR = COLS / E, ITER = LPR / 2;  // lanes a row, instructions
+    constexpr int B = ITER % 8 == 0 ? 8 : ITER % 4 == 0 ? 4 : 2;  // of a batch
+    static_assert(ITER % B == 0, "whole batches");
+    const int lane = threadIdx.x & 63;
+    asm volatile("" ::: "memory");  // the other lanes' rows, in the wave's own order
+    for (int p0 = 0; p0 < ITER; p0 += B) {
+        Out v[B];
+#pragma unroll
+        for (int p = 0; p < B; ++p) {
+            const int id = (p0 + p) * 64 + lane;
+            v[p] = *reinterpret_cast<const Out*>(stage + id / LPR * (2 * COLS + 16) + 2 * E * (id % LPR));
+        }
+#pragma unroll
+        for (int p = 0; p < B; ++p) {
+            const int id = (p0 + p) * 64 + lane, r = id / LPR, c = id % LPR * E;
+            uint16_t* out = dst + (int64_t)r * ldy + c;
+            if (r < rows && c + E <= left) {
+                *reinterpret_cast<Out*>(out) = v[p];
+            } else if (r < rows) {
+#pragma unroll
+                for (int e = 0; e + 1 < E; ++e)
+                    if (c + e < left) out[e] = v[p][e];
+            }
+        }
+    }
+    asm volatile("" ::: "memory");
 }
 
 // Position of chunk ch of row r in a row of CH chunks.
@@ -162,7 +208,7 @@ struct Grid {
     int mtiles, nblocks, per, splits;
     int group_m;  // tile rows walked together (x and W rows shared in an XCD's L2)
     int ldp;      // row stride of the partials
-    int wide;     // y's 8-column groups start on 16 bytes (1) or 8 (4); bias's on 16 (2)
+    int wide;     // y's rows start on 16 bytes (1), 8 (4) or 4 (8); bias on 16 (2)
 };
 
 // Requirements (checked by the launcher): x, w 16-byte aligned; K % 8 == 0
@@ -399,14 +445,61 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
     // ---- epilogue: lane (h, l32) of fragment (i, j) holds row
     // m0 + 32 (wm MT + i) + l32 and tile columns 32-block + 16 h + [0, 16)
     // (SWIGLU: outputs 16-block + 8 h + [0, 8)).
-    constexpr int OW = SWIGLU ? 8 : 16;  // outputs of a lane and fragment
+    constexpr int OW = SWIGLU ? 8 : 16, COLS = C::NT * 2 * OW;  // outputs of a lane and fragment, columns of a wave
     const int lim = min(n0 + gr.per, SWIGLU ? N >> 1 : N);
+    auto outputs = [&](uint32_t (&o)[OW / 2], int i, int j, int col) __attribute__((always_inline)) {
+        if constexpr (SWIGLU) {
+            uint32_t gu[8];
+            uint16_t v[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) gu[r] = pack_bf16x2(f32x2{acc[i][j][r], acc[i][j][r + 8]});
+            swiglu_bf16_batch<8>(gu, v);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = (uint32_t)v[2 * r] | ((uint32_t)v[2 * r + 1] << 16);
+        } else {
+#pragma unroll
+            for (int r = 0; r < 8; ++r) o[r] = pack_bf16x2(f32x2{acc[i][j][2 * r], acc[i][j][2 * r + 1]});
+            if (bias) {
+                add_bias8(o, bias, col, lim, gr.wide & 2);
+                add_bias8(o + 4, bias, col + 8, lim, gr.wide & 2);
+            }
+        }
+    };
+    if constexpr (C::STAGED) {
+        if (!(gr.wide & C::DIRECT) && gr.splits == 1) {
+            uint8_t* own = smem + wave % (C::WM * C::WN) * C::STORE_BYTES;
+            const int cb = n0 + wn * COLS;
+#pragma unroll
+            for (int i = 0; i < C::MT; ++i) {
+                const int mb = m0 + wm * (C::BM / C::WM) + 32 * i;
+                if (mb >= M || cb >= lim) break;
+#pragma unroll
+                for (int j = 0; j < C::NT; ++j) {
+                    const int col = cb + j * 2 * OW + OW * h;
+                    if (col >= lim) continue;
+                    uint32_t o[OW / 2];
+                    outputs(o, i, j, col);
+                    u32x4* dst = reinterpret_cast<u32x4*>(own + l32 * (2 * COLS + 16) + 2 * (col - cb));
+#pragma unroll
+                    for (int q = 0; q < OW / 8; ++q) dst[q] = u32x4{o[4 * q], o[4 * q + 1], o[4 * q + 2], o[4 * q + 3]};
+                }
+                uint16_t* dst = y + (int64_t)mb * ldy + cb;
+                if (gr.wide & 4)
+                    store_staged<4, COLS>(dst, ldy, own, min(32, M - mb), lim - cb);
+                else if (gr.wide & 8)
+                    store_staged<2, COLS>(dst, ldy, own, min(32, M - mb), lim - cb);
+                else
+                    store_staged<1, COLS>(dst, ldy, own, min(32, M - mb), lim - cb);
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < C::MT; ++i) {
         const int m = m0 + wm * (C::BM / C::WM) + 32 * i + l32;
 #pragma unroll
         for (int j = 0; j < C::NT; ++j) {
-            const int col = n0 + (wn * C::NT + j) * 2 * OW + OW * h;
+            const int col = n0 + wn * COLS + j * 2 * OW + OW * h;
             if (m >= M || col >= lim) continue;
             if constexpr (!SWIGLU) {
                 if (gr.splits > 1) {
@@ -420,22 +513,7 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
                 }
             }
             uint32_t o[OW / 2];
-            if constexpr (SWIGLU) {
-                uint32_t gu[8];
-                uint16_t v[8];
-#pragma unroll
-                for (int r = 0; r < 8; ++r) gu[r] = pack_bf16x2(f32x2{acc[i][j][r], acc[i][j][r + 8]});
-                swiglu_bf16_batch<8>(gu, v);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) o[r] = (uint32_t)v[2 * r] | ((uint32_t)v[2 * r + 1] << 16);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 8; ++r) o[r] = pack_bf16x2(f32x2{acc[i][j][2 * r], acc[i][j][2 * r + 1]});
-                if (bias) {
-                    add_bias8(o, bias, col, lim, gr.wide & 2);
-                    add_bias8(o + 4, bias, col + 8, lim, gr.wide & 2);
-                }
-            }
+            outputs(o, i, j, col);
             uint16_t* dst = y + (int64_t)m * ldy + col;
 #pragma unroll
             for (int q = 0; q < OW / 8; ++q) store8(dst + 8 * q, o + 4 * q, lim - col - 8 * q, gr.wide);
@@ -454,25 +532,17 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
     if (idx >= (int64_t)M * groups) return;
     const int m = (int)(idx / groups), col = 8 * (int)(idx % groups);
     const int64_t stride = (int64_t)M * ldp;
-    // D % 8 != 0: up's groups start off the 16-byte grid
+    // D % 4 != 0: up's groups start off the 16-byte grid
+    typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
     auto sum8 = [&](int c, float (&v)[8]) __attribute__((always_inline)) {
         const float* p = part + (int64_t)m * ldp + c;
-        if ((c & 3) == 0) {
-            f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
-            for (int s = 1; s < splits; ++s) {
-                a += *reinterpret_cast<const f32x4*>(p + s * stride);
-                b += *reinterpret_cast<const f32x4*>(p + s * stride + 4);
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = a[r], v[4 + r] = b[r];
-        } else {
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const int cc = c + r < N ? r : 0;
-                v[r] = p[cc];
-                for (int s = 1; s < splits; ++s) v[r] += p[s * stride + cc];
-            }
+        f32x4 a = *reinterpret_cast<const f32x4_any*>(p), b = *reinterpret_cast<const f32x4_any*>(p + 4);
+        for (int s = 1; s < splits; ++s) {
+            a += *reinterpret_cast<const f32x4_any*>(p + s * stride);
+            b += *reinterpret_cast<const f32x4_any*>(p + s * stride + 4);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = a[r], v[4 + r] = b[r];
     };
     float a[8];
     uint32_t o[4];

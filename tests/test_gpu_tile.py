@@ -58,12 +58,29 @@ def test_bf16_tile_output_stride_and_unaligned(fp8lin, gpu, oracle):
     assert_parity(bits(fp8lin.gemm_bf16(xs, up(w, gpu))), ref, "unaligned x")
 
 
+@pytest.mark.parametrize("off,extra", [(0, 4), (4, 4), (2, 2), (6, 12), (1, 0), (3, 13), (8, 8)])
+@pytest.mark.parametrize("m,n,k", [(9, 264, 40), (70, 312, 264), (129, 17416, 40), (515, 264, 1160), (1036, 4312, 72),
+                                   (2050, 4096, 136), (2050, 6664, 136)])
+def test_tile_output_rows_off_16_bytes(fp8lin, gpu, m, n, k, off, extra):
+    """Output rows that start on 8, 4 or 2 bytes (staged stores) hold the bits of
+    the aligned call, with nothing written beside them."""
+    rng = np.random.default_rng(m + n + k)
+    x, w = up(rand_bf16(rng, (m, k)), gpu), up(rand_bf16(rng, (n, k), 0.05), gpu)
+    ref = fp8lin.gemm_bf16(x, w)
+    for cols in (n, n - 3):
+        wide = torch.full((m, off + n + extra), 7.0, dtype=torch.bfloat16, device=gpu)
+        fp8lin.gemm_bf16(x, w[:cols], out=wide[:, off:off + cols])
+        part = wide[:, off:off + cols]
+        assert torch.equal(part, ref[:, :cols]) if cols == n else (part.float() - ref[:, :cols].float()).abs().max() < 0.1
+        assert (wide[:, :off] == 7).all() and (wide[:, off + cols:] == 7).all()
+
+
 # The FP8 tiles (32x32, 64x32, 64x64, 96x64, 128x64, 64x128, 96x192, 128x128
 # with K over two waves and at two per CU, 256x256) and K ranges of unequal
 # length.  K % 256 != 0 keeps the calls off the persistent GEMM.
 FP8_TILES = [(9, 261, 48), (70, 1030, 1168), (40, 4100, 400), (70, 4100, 144), (100, 8195, 272), (96, 16000, 144),
              (33, 17412, 144), (129, 17412, 48), (520, 4096, 1168), (513, 8195, 144), (1030, 12290, 144), (9, 261, 4112),
-             (65, 4100, 4112)]
+             (65, 4100, 4112), (300, 8200, 144), (150, 4120, 400)]
 
 
 @pytest.mark.parametrize("m,n,k", FP8_TILES)
