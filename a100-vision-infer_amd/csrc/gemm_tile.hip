@@ -21,12 +21,12 @@ struct Tile {
     int bm, bn, slots;
     float tau, tau1;
     LaunchFn plain, swiglu;
-    int (*lds)(int, int, int);
+    int lds;
 };
 
 template <class C, bool FP8>
 constexpr Tile tile(int slots, float tau, float tau1) {
-    return {C::BM, C::BN, slots, tau, tau1, gemm_tile::launch<C, false>, FP8 ? gemm_tile::launch<C, FP8> : nullptr, C::lds_bytes};
+    return {C::BM, C::BN, slots, tau, tau1, gemm_tile::launch<C, false>, FP8 ? gemm_tile::launch<C, FP8> : nullptr, C::LDS_BYTES};
 }
 
 // BF16 weights, M x N x K in us (torch's mm, hipBLASLt, beside it): 1036 x 3456
@@ -84,7 +84,7 @@ int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 float estimate(const Tile& t, int S, int M, int N, int K, int splits, int cus) {
     const int64_t units = (int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn) * splits;
     const float steps = (float)ceil_div(ceil_div(K, 128), splits), fixed = 2.0f + 6.0f * (float)(t.bm * t.bn) / 65536.0f;
-    const int slots = 2 * t.lds(S, K, splits) <= gemm_tile::kLds ? t.slots : 1;
+    const int slots = 2 * t.lds <= gemm_tile::kLds ? t.slots : 1;
     const float tau = slots < t.slots ? t.tau1 : t.tau;
     const int64_t whole = units / ((int64_t)cus * slots), rest = units - whole * cus * slots;
     float us = 2.0f + (float)whole * (fixed + steps * tau);
@@ -140,7 +140,6 @@ TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split) {
         const int64_t tiles = (int64_t)ceil_div(M, t.bm) * ceil_div(N, t.bn);
         const int most = may_split ? std::min(kMaxTileSplits, ceil_div(K, 128)) : 1;
         for (int s = 1; s <= most && (s == 1 || tiles * s <= cus); ++s) {
-            if (t.lds(S, K, s) > gemm_tile::kLds) continue;
             const float us = estimate(t, S, M, N, K, s, cus);
             if (best.cfg < 0 || us < best.us) best = {i, s, us};
         }

@@ -35,14 +35,6 @@ using gemm_fp8::make_desc;
 
 constexpr int kLds = 160 * 1024;
 
-// 128-K scale blocks that a K range of kt steps may touch.
-template <class C>
-__host__ __device__ inline int scale_blocks(int S, int kt) {
-    if (S == 1) return 1;
-    const int b = kt * C::BK / 128 + (C::BK < 128 ? 2 : 1);
-    return b < S ? b : S;
-}
-
 // PIPE: the next slice's fragments are read (and dequantized) into a second
 // register set while the current ones are multiplied; stage t + 1 must then
 // have landed before step t, one stage less in flight.  It gains 5-8% where a
@@ -67,6 +59,21 @@ struct Cfg {
     static_assert(X_STAGE % (1024 * WAVES) == 0 && W_STAGE % (1024 * WAVES) == 0, "equal DMA shares");
     static_assert(WK == 1 || BM * BN * 4 <= RING, "a partial tile fits the ring");
     static_assert(RING <= kLds, "LDS");
+    // Waves per SIMD to leave registers for: a workgroup's own, or as many as the
+    // 128x128 FP8 tile of four waves has in LDS (two of them: 10% slower).
+    static constexpr int EU = FP8 && WAVES == 4 && RING <= kLds / 3 ? kLds / RING : (WAVES + 3) / 4;
+    // FP8: the rows' scales, in two windows of SWB 128-K blocks beside the ring:
+    // while the SPW steps of one run, SQ DMAs a wave fill the other.  Scales of
+    // the whole K in LDS left no room for the large tiles at K above 8064
+    // (256x256): 1016 x 29884 x 11392 took 1074 us in smaller ones, 737 now.
+    // A DMA's 256 bytes hold 64 / SWB rows; the next ones start on another bank,
+    // so that 32 rows at one block fall in distinct banks.
+    static constexpr int SWB = BK == 128 ? 8 : 4, SPW = SWB * 128 / BK, SQ = FP8 ? BN * SWB / 64 / WAVES : 0;
+    static constexpr int SCHUNK = 260, SWIN = BN * SWB / 64 * SCHUNK;
+    static constexpr int LDS_BYTES = RING + (FP8 ? 2 * SWIN : 0);
+    static_assert(!FP8 || BN * SWB % (64 * WAVES) == 0, "equal scale DMA shares");
+    static_assert(ST <= SPW && SPW % 2 == 0, "a window's scales, issued in the one before, land before its first step");
+    static_assert(LDS_BYTES <= kLds, "LDS");
     // Output rows off the 16-byte grid go through LDS (store_staged), in the part
     // of the ring that each wave then has to itself; 4 is rows on 8 bytes, which
     // the smaller tiles store as they are.  Lane's own rows and staged, us: 512 x
@@ -77,12 +84,6 @@ struct Cfg {
     static constexpr int DIRECT = BM * BN >= 128 * 128 ? 1 : 1 | 4;
     static constexpr int STORE_BYTES = WK > 1 ? MT * NT * 4096 : 32 * (NT * 64 + 16);
     static_assert(!STAGED || (STORE_BYTES >= 32 * (NT * 64 + 16) && WM * WN * STORE_BYTES <= RING), "32 rows of a wave's tile");
-    // Ring and, for FP8, the rows' scales of the longest K range, padded to an
-    // odd stride so that 32 rows at one block fall in distinct banks.
-    static int lds_bytes(int S, int K, int splits) {
-        const int ksteps = (K + BK - 1) / BK, kt = (ksteps + splits - 1) / splits;
-        return RING + (FP8 ? BN * (scale_blocks<Cfg>(S, kt) | 1) * 4 : 0);
-    }
 };
 
 // o = bf16(y + bias) of eight rounded outputs from column c on, as the separate
@@ -178,9 +179,20 @@ __device__ __forceinline__ void wait_vm_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
 }
 
+// 64 lanes x 4 B from global (voff + soff, bounds-checked) into LDS
+// [m0v, m0v + 256), lane l at m0v + 4 l.
+__device__ __forceinline__ void dma4(uint32_t m0v, uint32_t voff, i32x4 desc, int soff) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 ::"s"(m0v), "v"(voff), "s"(desc), "s"(soff) : "memory", "m0");
+}
+
 // 16-byte chunk at LDS byte address a.
 __device__ __forceinline__ u32x4 lds16(uint32_t a) {
     return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)a);
+}
+
+__device__ __forceinline__ float lds4(uint32_t a) {
+    return *reinterpret_cast<const __attribute__((address_space(3))) float*>((uintptr_t)a);
 }
 
 // Weight row of tile row b (fragment order) of the column block that starts at
@@ -216,7 +228,7 @@ struct Grid {
 // 2^31; S == 1 or ceil(K / 128); per % 8 == 0 and per <= BN (SWIGLU: BN / 2).
 // With SWIGLU, N counts weight rows and y is [M, N/2].
 template <class C, bool SWIGLU>
-__global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
+__global__ __launch_bounds__(C::THREADS, C::EU) void gemm_tile_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
                                                                const float* __restrict__ scales, int S,
                                                                const uint16_t* __restrict__ bias,
                                                                uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K,
@@ -265,6 +277,19 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
     }
     const uint32_t m0x = __builtin_amdgcn_readfirstlane(lds0 + wave * C::XD * 1024);
     const uint32_t m0w = __builtin_amdgcn_readfirstlane(lds0 + C::X_STAGE + wave * C::WD * 1024);
+    // FP8: scale DMA q of this wave fills 64 / SWB rows of a window: lane l ->
+    // row l / SWB, block l % SWB.  The range's step 0 is step tt0 of window 0.
+    // Row scales are block 0 of window 0, which nothing overwrites.
+    const int kb0 = S == 1 ? 0 : (t0 * C::BK) >> 7, tt0 = t0 % (128 / C::BK);
+    const i32x4 ds = make_desc(scales, C::FP8 ? (uint32_t)((int64_t)N * S * 4) : 0u);
+    uint32_t soff[C::FP8 ? C::SQ : 1];
+    const int sblk = kb0 + lane % C::SWB;
+    const uint32_t m0s = __builtin_amdgcn_readfirstlane(lds0 + C::RING + wave * C::SQ * C::SCHUNK);
+    auto scale_window = [&](int wd) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < C::SQ; ++q)
+            dma4(m0s + (wd & 1) * C::SWIN + q * C::SCHUNK, sblk + wd * C::SWB < S ? soff[q] + (uint32_t)(wd * C::SWB * 4) : kBufferOob, ds, 0);
+    };
     auto issue = [&](int t, uint32_t slot) __attribute__((always_inline)) {
         // past the range's last step: nothing (the same number of DMAs)
         const int k = (t0 + t) * C::BK, kend = t < KT ? K : 0;
@@ -275,16 +300,13 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
         for (int d = 0; d < C::WD; ++d)
             dma16(m0w + slot + d * 1024, k + wk0[d] < kend ? woff[d] : kBufferOob, dw, C::FP8 ? k : k * 2);
     };
-    // FP8: the tile's scales of this K range in fragment row order, [BN][stride].
-    float* sc = reinterpret_cast<float*>(smem + C::RING);
-    const int kb0 = S == 1 ? 0 : (t0 * C::BK) >> 7, SB = scale_blocks<C>(S, KT);
-    const int sstride = SB | 1;
     if constexpr (C::FP8) {
-        for (int i = threadIdx.x; i < C::BN * SB; i += C::THREADS) {
-            const int r = i / SB, c = i - r * SB;
-            const int64_t n = weight_row<SWIGLU>(n0, gr.per, r, N);
-            sc[r * sstride + c] = n >= 0 && kb0 + c < S ? scales[n * S + kb0 + c] : 0.0f;
+#pragma unroll
+        for (int q = 0; q < C::SQ; ++q) {
+            const int64_t n = weight_row<SWIGLU>(n0, gr.per, (wave * C::SQ + q) * (64 / C::SWB) + lane / C::SWB, N);
+            soff[q] = n >= 0 ? (uint32_t)((n * S + sblk) * 4) : kBufferOob;
         }
+        scale_window(0);
     }
 #pragma unroll
     for (int p = 0; p < C::ST - 1; ++p) issue(p, p * C::STAGE);
@@ -300,22 +322,29 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
     // Fragment row bases; the swizzle of a row depends on the row mod 16 only.
     const uint32_t xrow = lds0 + (wm * (C::BM / C::WM) + l32) * C::XROW;
     const uint32_t wrow = lds0 + C::X_STAGE + (wn * (C::BN / C::WN) + l32) * C::WROW;
-    const float* srow = sc + (wn * (C::BN / C::WN) + l32) * sstride;
+    const uint32_t srow = lds0 + C::RING + l32 / (64 / C::SWB) * C::SCHUNK + l32 % (64 / C::SWB) * C::SWB * 4 +
+                          wn * (C::BN / C::WN / 32) * (C::SWB / 2) * C::SCHUNK;
     // A slice of 32 K: lane half h holds K [16 h, 16 h + 16) of it, its first
     // 8 in the first MFMA and the rest in the second, for x and W alike.
     constexpr int SETS = C::PIPE ? 2 : 1;
     u32x4 a[SETS][C::NT][2], b[SETS][C::MT][2], raw[C::NT];
     float scl[C::NT];
     const int klim = K - 16 * h;
-    auto fetch = [&](int set, uint32_t stage, int s, int t) __attribute__((always_inline)) {
+    // Byte offset of step t's scale block in the windows.
+    auto scale_at = [&](int t) __attribute__((always_inline)) {
+        const uint32_t kb = S == 1 ? 0u : (uint32_t)(t + tt0) * C::BK / 128;  // block within the range
+        return (kb / C::SWB & 1) * C::SWIN + kb % C::SWB * 4;
+    };
+    // MASK: K may end in this step.  sa: scale_at(t), worked out a step ahead, and
+    // the scales are read first: the conversions wait for them.
+    auto fetch = [&]<bool MASK>(int set, uint32_t stage, int s, int t, uint32_t sa) __attribute__((always_inline)) {
         if constexpr (C::FP8) {
-            const int kb = S == 1 ? 0 : min((((t0 + t) * C::BK) >> 7) - kb0, SB - 1);
-            // a chunk past K holds zero codes; its scale must be zero too (0 * inf)
-            const bool in_k = (t0 + t) * C::BK + 32 * s < klim;
 #pragma unroll
             for (int j = 0; j < C::NT; ++j) {
+                scl[j] = lds4(srow + sa + j * (C::SWB / 2) * C::SCHUNK);
                 raw[j] = lds16(wrow + stage + j * 32 * C::WROW + 16 * swz<CHW>(l32, 2 * s + h));
-                scl[j] = in_k ? srow[j * 32 * sstride + kb] : 0.0f;
+                // a chunk past K holds zero codes; its scale must be zero too (0 * inf)
+                if constexpr (MASK) scl[j] = (t0 + t) * C::BK + 32 * s < klim ? scl[j] : 0.0f;
             }
         } else {
 #pragma unroll
@@ -356,53 +385,97 @@ __global__ __launch_bounds__(C::THREADS) void gemm_tile_kernel(const uint16_t* _
                                                                         acc[i][j], 0, 0, 0);
     };
     constexpr int SL = C::SLICES / C::WK;  // slices of a wave per step
+    uint32_t sa = C::FP8 ? scale_at(0) : 0u, sn = C::FP8 ? scale_at(1) : 0u;  // of this step and the next
     uint32_t rd = 0, nx = C::STAGE, wr = (C::ST - 1) * C::STAGE;
     auto next = [&](uint32_t v) __attribute__((always_inline)) { return v == (C::ST - 1) * C::STAGE ? 0u : v + C::STAGE; };
+    // Steps that need no mask (PIPE: step t also fetches from step t + 1).
+    const int plain = C::FP8 && (t0 + KT) * C::BK > K ? max(KT - (C::PIPE ? 2 : 1), 0) : KT;
+    // Runs body(first, last) over the steps [0, plain), with window w + 1's
+    // scale DMAs between two of them: behind the barrier of window w's first
+    // step, where every wave is done with window w - 1.  (Asked for in every
+    // step, the same DMAs cost the loop 7 to 10% of its time.)  They come on
+    // top of the ND a step that the waits count, which only makes those wait
+    // for no less than they should.  An even step for PIPE's pairs.
+    auto windows = [&](auto body) __attribute__((always_inline)) {
+        if constexpr (!C::FP8) {
+            body(0, plain);
+        } else {
+            const int at = C::PIPE ? 2 - 2 * tt0 : 1 - tt0;
+            int t = 0;
+            for (int w = 0;; ++w) {
+                const int stop = S == 1 ? plain : min(plain, at + w * C::SPW);
+                body(t, stop);
+                if (stop == plain) break;
+                t = stop;
+                scale_window(w + 1);
+            }
+        }
+    };
     if constexpr (C::PIPE) {
         static_assert(SL == 1 || SL % 2 == 0, "register sets alternate");
         // Step t: stages t and t + 1 have landed for every wave, and every
         // wave is done reading stage t - 1, whose slot takes stage t + ST - 1.
-        auto step = [&](int t, int p) __attribute__((always_inline)) {
+        auto step = [&]<bool MASK>(int t, int p) __attribute__((always_inline)) {
             wait_vm_barrier<(C::ST - 3) * C::ND>();
             issue(t + C::ST - 1, wr);
 #pragma unroll
             for (int s0 = 0; s0 < SL; ++s0) {
                 const int cur = (p + s0) & 1;
                 if (s0 + 1 < SL)
-                    fetch(cur ^ 1, rd, (s0 + 1) * C::WK + wk, t);
+                    fetch.template operator()<MASK>(cur ^ 1, rd, (s0 + 1) * C::WK + wk, t, sa);
                 else
-                    fetch(cur ^ 1, nx, wk, t + 1);
+                    fetch.template operator()<MASK>(cur ^ 1, nx, wk, t + 1, sn);
                 multiply(cur);
                 convert(cur ^ 1);
             }
             rd = nx;
             nx = next(nx);
             wr = next(wr);
+            sa = sn;
+            if constexpr (C::FP8) sn = scale_at(t + 2);
         };
         wait_vm_barrier<(C::ST - 2) * C::ND>();
-        fetch(0, rd, wk, 0);
+        fetch.template operator()<true>(0, rd, wk, 0, sa);
         convert(0);
+        int t = 0;
         if constexpr (SL == 1) {
-            for (int t = 0; t < KT; t += 2) {
-                step(t, 0);
-                if (t + 1 < KT) step(t + 1, 1);
+            windows([&](int first, int last) __attribute__((always_inline)) {
+                for (t = first; t + 1 < last; t += 2) {
+                    step.template operator()<false>(t, 0);
+                    step.template operator()<false>(t + 1, 1);
+                }
+            });
+            for (; t < KT; t += 2) {
+                step.template operator()<C::FP8>(t, 0);
+                if (t + 1 < KT) step.template operator()<C::FP8>(t + 1, 1);
             }
         } else {
-            for (int t = 0; t < KT; ++t) step(t, 0);
+            windows([&](int first, int last) __attribute__((always_inline)) {
+                for (t = first; t < last; ++t) step.template operator()<false>(t, 0);
+            });
+            if constexpr (C::FP8)
+                for (; t < KT; ++t) step.template operator()<true>(t, 0);
         }
     } else {
-        for (int t = 0; t < KT; ++t) {
+        auto step = [&]<bool MASK>(int t) __attribute__((always_inline)) {
             wait_vm_barrier<(C::ST - 2) * C::ND>();
             issue(t + C::ST - 1, wr);
 #pragma unroll
             for (int s0 = 0; s0 < SL; ++s0) {
-                fetch(0, rd, s0 * C::WK + wk, t);
+                fetch.template operator()<MASK>(0, rd, s0 * C::WK + wk, t, sa);
                 convert(0);
                 multiply(0);
             }
             rd = next(rd);
             wr = next(wr);
-        }
+            if constexpr (C::FP8) sa = scale_at(t + 1);
+        };
+        int t = 0;
+        windows([&](int first, int last) __attribute__((always_inline)) {
+            for (t = first; t < last; ++t) step.template operator()<false>(t);
+        });
+        if constexpr (C::FP8)
+            if (t < KT) step.template operator()<true>(t);
     }
     // The last steps prefetched zeros past K; they must land before the ring
     // is reused or the workgroup's LDS is freed.
@@ -579,7 +652,7 @@ hipError_t launch(const uint16_t* x, const void* w, const float* scales, int S, 
     static const hipError_t attr = allow_lds(reinterpret_cast<const void*>(kern), kLds);
     if (attr != hipSuccess) return attr;
     const int units = gr.mtiles * gr.nblocks * gr.splits;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((units + 7) / 8 * 8)), dim3(C::THREADS), C::lds_bytes(S, K, gr.splits), stream,
+    hipLaunchKernelGGL(kern, dim3((unsigned)((units + 7) / 8 * 8)), dim3(C::THREADS), C::LDS_BYTES, stream,
                        x, w, scales, S, bias, y, ldy, M, N, K, gr, part);
     return hipGetLastError();
 }

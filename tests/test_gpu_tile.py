@@ -103,6 +103,26 @@ def test_fp8_tile(fp8lin, gpu, oracle, m, n, k, rows_scaled):
             assert torch.equal(fp8lin.linear_swiglu(xd, cd, sd, split=split), fp8lin.fused_swiglu(y))
 
 
+@pytest.mark.parametrize("m,n,k", [(9, 8195, 2320), (33, 4100, 2192), (97, 8200, 3248), (129, 16400, 1808), (200, 16400, 1168),
+                                   (513, 21000, 1168), (300, 2304, 9296), (65, 4100, 9296)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_tile_long_k(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """K over several windows of scales, ending inside a step, whole and in K
+    ranges that start inside a block: a column sample against the oracle, with
+    scales that differ by powers of two from block to block."""
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    shape = n if rows_scaled else (n, (k + 127) // 128)
+    scales = np.exp2(-rng.integers(6, 12, shape)).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    rows, cols = sample(m), np.r_[0:33, n // 2:n // 2 + 33, n - 33:n]
+    ref = oracle.linear(x[rows], codes[cols], scales[cols])
+    for split in (False, True):
+        y = fp8lin.fp8_linear(xd, cd, sd, split=split)
+        assert_parity(bits(y)[rows][:, cols], ref, f"long K {m}x{n}x{k} split={split}")
+
+
 @pytest.mark.parametrize("m,n,k", FP8_TILES)
 @pytest.mark.parametrize("rows_scaled", [False, True])
 def test_fp8_tile_infinite_scale(fp8lin, gpu, m, n, k, rows_scaled):
