@@ -1,8 +1,9 @@
 // Prefill GEMM dispatch.  FP8 weights with K % 256 == 0 run gemm_fp8_kernel
 // (gemm_fp8.hpp) or, where its estimate is lower, one tile per workgroup
 // (gemm_tile.hip); other K whose rows start on 16 bytes and BF16 weights run
-// the tiles, and what is left (unaligned operands, K off the 16-byte grid,
-// 2 GiB operands) the general template of gemm_kernel.hpp.
+// the tiles, the largest FP8 ones by the template of gemm_kernel.hpp where K %
+// 64 == 0, and what is left (unaligned operands, K off the 16-byte grid, 2 GiB
+// operands) that template with element-wise loads.
 #include <algorithm>
 #include <atomic>
 
@@ -15,10 +16,21 @@ namespace {
 
 constexpr int kGroupM = 8;  // XCD-local tile patch height
 
+using Block = gemm::Cfg<256, 256, 64, 2, 4>;
+
+// The template with element-wise loads.
 template <bool FP8, bool SWIGLU>
-hipError_t run(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y,
+hipError_t run(const uint16_t* x, const void* w, const float* scales, int S, const uint16_t* bias, uint16_t* y,
                int64_t ldy, int M, int N, int K, hipStream_t stream) {
-    return gemm::launch<gemm::Cfg<256, 256, 64, 2, 4>, FP8, SWIGLU, kGroupM>(x, w, scales, S, y, ldy, M, N, K, stream);
+    return gemm::launch<Block, FP8, true, SWIGLU, kGroupM, 1>(x, w, scales, S, bias, y, ldy, M, N, K, stream);
+}
+
+// The template with 16-byte loads two K steps ahead, the next stage's
+// dequantization and LDS store after the second MFMA group.
+template <bool SWIGLU>
+hipError_t run_block(const uint16_t* x, const void* w, const float* scales, int S, const uint16_t* bias, uint16_t* y,
+                     int64_t ldy, int M, int N, int K, hipStream_t stream) {
+    return gemm::launch<Block, true, false, SWIGLU, kGroupM, 1, 2, 1>(x, w, scales, S, bias, y, ldy, M, N, K, stream);
 }
 
 // Work plan of the persistent FP8 GEMM (see gemm_fp8.hpp).  Without a
@@ -223,18 +235,22 @@ float estimate(const gemm_fp8::Plan& p, int K, int G) {
 // How an FP8 call of more than 8 rows that is neither skinny nor mid rows
 // runs: the persistent GEMM under `plan`, the tiles under `tile`, or (neither)
 // the general template.  have: the bytes of workspace that K-split partials
-// may take; a plan that needs more is made without a split.  The persistent
+// may take; a plan that needs more is made without a split.  block: the
+// template's 256x256 tiles in the place of gemm_tile.hip's, where K allows and
+// they are one round on more than 0.6 of the CUs: 4096 x 2560 x 13440 316 us
+// against 345, 1036 x 8944 x 5248 129 against 141; median of 80 such shapes
+// 0.97, and 1.05 on fewer CUs, 1.03 over more rounds.  The persistent
 // GEMM's unsplit sums do not depend on the row count or the tile height, and
 // the entry points that take no workspace (any false) keep them: there the
 // tiles only run the K that it does not.
 struct Route {
-    bool gemm, tiles;
+    bool gemm, tiles, block;
     gemm_fp8::Plan plan;
     TilePlan tile;
 };
 
 Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, int K, bool swiglu, bool any, size_t have) {
-    Route r{fp8_kernel_ok(x, w, S, ldy, M, N, K), false, {}, {}};
+    Route r{fp8_kernel_ok(x, w, S, ldy, M, N, K), false, false, {}, {}};
     const int G = compute_units();
     // 192-row tiles, unsplit, where their round is the cheaper one: 256-row
     // tiles that fill half the CUs to two thirds, or are half padding.  M x N x
@@ -256,6 +272,8 @@ Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, 
         r.tiles = r.tile.cfg >= 0 && (!r.gemm || r.tile.us < 0.95f * estimate(fitting(false), K, G));
     }
     if (r.tiles) r.gemm = false;
+    const int64_t blocks = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+    r.block = r.tiles && tile_is_block(r.tile) && gemm::aligned(x, w, true, M, N, K) && blocks <= G && 10 * blocks > 6 * G;
     return r;
 }
 
@@ -284,6 +302,11 @@ hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales,
     const Route r = route(x, w, S, ldy, M, N, K, swiglu, may_split, have);
     if (r.gemm && r.plan.rtiles == 0 && halves(x, w, S, M, N, K))
         return launch_halves(x, codes, scales, y, ldy, M, N, K, swiglu, stream);
+    if (r.block) {
+        if (bias) *bias_added = true;
+        return swiglu ? run_block<true>(x, w, scales, S, nullptr, y, ldy, M, N, K, stream)
+                      : run_block<false>(x, w, scales, S, bias, y, ldy, M, N, K, stream);
+    }
     if (r.tiles) {
         if (bias) *bias_added = true;
         return launch_tile(r.tile, true, x, w, scales, S, bias, y, ldy, M, N, K, swiglu, ws, stream);
@@ -294,8 +317,9 @@ hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales,
         return swiglu ? run_fp8<true>(x, codes, scales, S, y, ldy, M, N, K, r.plan, G, part, stream)
                       : run_fp8<false>(x, codes, scales, S, y, ldy, M, N, K, r.plan, G, part, stream);
     }
-    return swiglu ? run<true, true>(x, w, scales, S, y, ldy, M, N, K, stream)
-                  : run<true, false>(x, w, scales, S, y, ldy, M, N, K, stream);
+    if (bias) *bias_added = true;
+    return swiglu ? run<true, true>(x, w, scales, S, nullptr, y, ldy, M, N, K, stream)
+                  : run<true, false>(x, w, scales, S, bias, y, ldy, M, N, K, stream);
 }
 
 hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
@@ -303,8 +327,8 @@ hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t
     if (!skinny(M, N, false) && tile_supported(x, w, false, 1, M, N, K))
         return launch_tile(tile_plan(false, 1, M, N, K, false), false, x, w, nullptr, 1, bias, y, ldy, M, N, K, false,
                            nullptr, stream);
-    const hipError_t e = skinny(M, N, false) ? launch_skinny(x, w, nullptr, 1, y, ldy, M, N, K, false, stream)
-                                             : run<false, false>(x, w, nullptr, 1, y, ldy, M, N, K, stream);
+    if (!skinny(M, N, false)) return run<false, false>(x, w, nullptr, 1, bias, y, ldy, M, N, K, stream);
+    const hipError_t e = launch_skinny(x, w, nullptr, 1, y, ldy, M, N, K, false, stream);
     return e != hipSuccess || !bias ? e : launch_bias(y, ldy, bias, M, N, stream);
 }
 

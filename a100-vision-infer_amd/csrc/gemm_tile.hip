@@ -147,6 +147,8 @@ TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split) {
     return best;
 }
 
+bool tile_is_block(const TilePlan& p) { return p.splits == 1 && kFp8[p.cfg].bm == 256 && kFp8[p.cfg].bn == 256; }
+
 size_t tile_plan_bytes(const TilePlan& p, int M, int N) {
     return p.splits <= 1 ? 0 : (size_t)p.splits * M * (ceil_div(N, 8) * 8 + 8) * sizeof(float);
 }

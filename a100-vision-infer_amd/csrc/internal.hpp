@@ -76,6 +76,7 @@ struct TilePlan {
 bool tile_supported(const uint16_t* x, const void* w, bool fp8, int S, int64_t M, int64_t N, int64_t K);
 TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split);
 size_t tile_plan_bytes(const TilePlan& p, int M, int N);
+bool tile_is_block(const TilePlan& p);  // FP8, whole 256x256 tiles
 hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,
                        const uint16_t* bias, uint16_t* y, int64_t ldy, int M, int N, int K, bool swiglu, void* ws,
                        hipStream_t stream);

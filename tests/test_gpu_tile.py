@@ -123,6 +123,31 @@ def test_fp8_tile_long_k(fp8lin, gpu, oracle, m, n, k, rows_scaled):
         assert_parity(bits(y)[rows][:, cols], ref, f"long K {m}x{n}x{k} split={split}")
 
 
+@pytest.mark.parametrize("m,n,k", [(1036, 8944, 320), (512, 25090, 448), (466, 24578, 1216), (2048, 5382, 192)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_block_template(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """One round of 256x256 tiles on more than 0.6 of the CUs with K % 64 == 0:
+    against the oracle, fused SwiGLU equal to the plain form's, a bias added to
+    the rounded outputs, a row of NaN in its row."""
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random(n if rows_scaled else (n, (k + 127) // 128)) * .01 + .001).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    cd, sd, b = up(codes, gpu), up(scales, gpu), up(rand_bf16(rng, (n,)), gpu)
+    y = fp8lin.fp8_linear(up(x, gpu), cd, sd)
+    rows, cols = sample(m), np.r_[0:65, n - 65:n]
+    assert_parity(bits(y)[rows][:, cols], oracle.linear(x[rows], codes[cols], scales[cols]), f"block {m}x{n}x{k}")
+    assert torch.equal(fp8lin.linear_swiglu(up(x, gpu), cd, sd), fp8lin.fused_swiglu(y))
+    eng = fp8lin.LinearEngine()
+    eng.add("p.weight", cd, sd)
+    eng.add("p.bias", b)
+    assert torch.equal(eng.linear(up(x, gpu), "p"), fp8lin.add_bias(y.clone(), b))
+    x[m // 2] = 0x7fc0  # NaN
+    bad = fp8lin.fp8_linear(up(x, gpu), cd, sd)
+    keep = np.arange(m) != m // 2
+    assert torch.equal(bad[keep], y[keep]) and torch.isnan(bad[m // 2]).all()
+
+
 @pytest.mark.parametrize("m,n,k", FP8_TILES)
 @pytest.mark.parametrize("rows_scaled", [False, True])
 def test_fp8_tile_infinite_scale(fp8lin, gpu, m, n, k, rows_scaled):
