@@ -211,24 +211,24 @@ int compute_units() {
 
 namespace {
 
-// Estimated us of the persistent FP8 GEMM under plan p, from its measured
-// times: us per 256 K of a round of tiles, which grows with the share of the
-// CUs that run one (256-row tiles 4.3 at 0.53 of them, 5.0 at 0.80, 5.8 at
-// 0.98; 192-row tiles 3.7 at 0.66, 4.1 at 0.80, 4.8 at 0.98; whole rounds 6.1
-// and 5.0; 128-row tiles 3.8), and for a split the partials' round trip and
-// the second launch.
+// Estimated us of the persistent FP8 GEMM under plan p, fitted to 1900 calls of
+// it with weights from HBM (half of them within 4%, nine tenths within 13%): us
+// per 256 K of a round of tiles, which grows with the share of the CUs that run
+// one; for each round after the first its fill and drain; and for a split the
+// partials' round trip and the second launch.
 float estimate(const gemm_fp8::Plan& p, int K, int G) {
     const int chunks = K / 256, rounds = p.full / G;
     const float share = (float)(p.full - rounds * G) / (float)G;
-    const float round = p.bm == 128 ? 3.8f : p.bm == 192 ? 5.0f : 6.1f;
-    const float last = p.bm == 128   ? 3.8f
-                       : p.bm == 192 ? 3.7f + 3.3f * std::max(0.0f, share - 0.66f)
-                                     : 4.3f + 3.2f * std::max(0.0f, share - 0.53f);
-    float us = 5.0f + (float)chunks * ((float)rounds * round + (share > 0.0f ? last : 0.0f));
-    const float c = p.bm == 128 ? 3.8f : p.full >= G ? 6.1f : 4.8f;
+    const float round = p.bm == 128 ? 3.2f : p.bm == 192 ? 5.0f : 6.05f;
+    const float last = p.bm == 128   ? 3.3f + 2.0f * std::max(0.0f, share - 0.5f)
+                       : p.bm == 192 ? 3.5f + 5.5f * std::max(0.0f, share - 0.66f)
+                                     : 4.6f + 4.2f * std::max(0.0f, share - 0.53f);
+    float us = 7.2f + (float)chunks * ((float)rounds * round + (share > 0.0f ? last : 0.0f));
+    us += 8.0f * (float)std::max(0, rounds + (share > 0.0f) + (p.rtiles > 0) - 1);
+    const float c = p.bm == 128 ? 3.4f : p.full >= G ? 5.75f : 5.35f;
     if (p.rtiles > 0)
-        us += c * (float)((chunks + p.splits - 1) / p.splits) + 4.0f +
-              8.0e-6f / 5.2f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
+        us += c * (float)((chunks + p.splits - 1) / p.splits) + 1.15f +
+              0.95e-6f * (float)p.rtiles * (float)p.splits * (float)(p.bm * gemm_fp8::BN);
     return us;
 }
 
@@ -266,10 +266,10 @@ Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, 
     };
     if (r.gemm) r.plan = fitting(swiglu);
     if (tile_supported(x, w, true, S, M, N, K) && (!r.gemm || any)) {
-        r.tile = tile_plan(true, S, M, N, K, any);
-        if (tile_plan_bytes(r.tile, M, N) > have) r.tile = tile_plan(true, S, M, N, K, false);
+        r.tile = tile_plan(true, M, N, K, any);
+        if (tile_plan_bytes(r.tile, M, N) > have) r.tile = tile_plan(true, M, N, K, false);
         // against the plain form's plan for both epilogues: one route for both
-        r.tiles = r.tile.cfg >= 0 && (!r.gemm || r.tile.us < 0.95f * estimate(fitting(false), K, G));
+        r.tiles = (!r.gemm || r.tile.us < 0.95f * estimate(fitting(false), K, G));
     }
     if (r.tiles) r.gemm = false;
     const int64_t blocks = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
@@ -325,7 +325,7 @@ hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales,
 hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t* bias, uint16_t* y, int64_t ldy, int M,
                             int N, int K, hipStream_t stream) {
     if (!skinny(M, N, false) && tile_supported(x, w, false, 1, M, N, K))
-        return launch_tile(tile_plan(false, 1, M, N, K, false), false, x, w, nullptr, 1, bias, y, ldy, M, N, K, false,
+        return launch_tile(tile_plan(false, M, N, K, false), false, x, w, nullptr, 1, bias, y, ldy, M, N, K, false,
                            nullptr, stream);
     if (!skinny(M, N, false)) return run<false, false>(x, w, nullptr, 1, bias, y, ldy, M, N, K, stream);
     const hipError_t e = launch_skinny(x, w, nullptr, 1, y, ldy, M, N, K, false, stream);

@@ -596,8 +596,8 @@ __global__ __launch_bounds__(C::THREADS, C::EU) void gemm_tile_kernel(const uint
 
 // y = bf16(sum over splits, in order) (+ bias), or SWIGLU y = swiglu of the
 // gate and up sums: eight outputs per thread.
-template <bool SWIGLU>
-__global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part, int splits, int ldp,
+template <bool SWIGLU, int SPLITS>
+__global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restrict__ part, int ldp,
                                                            const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
                                                            int64_t ldy, int M, int N, int wide) {
     const int D = SWIGLU ? N >> 1 : N, groups = (D + 7) / 8;
@@ -609,13 +609,16 @@ __global__ __launch_bounds__(256) void split_reduce_kernel(const float* __restri
     typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
     auto sum8 = [&](int c, float (&v)[8]) __attribute__((always_inline)) {
         const float* p = part + (int64_t)m * ldp + c;
-        f32x4 a = *reinterpret_cast<const f32x4_any*>(p), b = *reinterpret_cast<const f32x4_any*>(p + 4);
-        for (int s = 1; s < splits; ++s) {
-            a += *reinterpret_cast<const f32x4_any*>(p + s * stride);
-            b += *reinterpret_cast<const f32x4_any*>(p + s * stride + 4);
+        f32x4 a[SPLITS], b[SPLITS];  // all under way before the first sum
+#pragma unroll
+        for (int s = 0; s < SPLITS; ++s) {
+            a[s] = *reinterpret_cast<const f32x4_any*>(p + s * stride);
+            b[s] = *reinterpret_cast<const f32x4_any*>(p + s * stride + 4);
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = a[r], v[4 + r] = b[r];
+        for (int s = 1; s < SPLITS; ++s) a[0] += a[s], b[0] += b[s];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = a[0][r], v[4 + r] = b[0][r];
     };
     float a[8];
     uint32_t o[4];

@@ -74,7 +74,7 @@ struct TilePlan {
     float us;  // estimated time
 };
 bool tile_supported(const uint16_t* x, const void* w, bool fp8, int S, int64_t M, int64_t N, int64_t K);
-TilePlan tile_plan(bool fp8, int S, int M, int N, int K, bool may_split);
+TilePlan tile_plan(bool fp8, int M, int N, int K, bool may_split);
 size_t tile_plan_bytes(const TilePlan& p, int M, int N);
 bool tile_is_block(const TilePlan& p);  // FP8, whole 256x256 tiles
 hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,
