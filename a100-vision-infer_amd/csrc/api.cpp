@@ -554,6 +554,18 @@ size_t fp8lin_linear_scaled_workspace_bytes(int64_t M, int64_t N, int64_t K, int
     return linear_ws(M, N, K, scale_cols, false);
 }
 
+int fp8lin_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t scale_cols, int split, int* plan) {
+    return guarded([&] {
+        require(plan != nullptr, FP8LIN_ERR_ARGUMENT, "GEMM plan: null pointer");
+        check_dims(M, N, K);
+        require(M > 8, FP8LIN_ERR_SHAPE, "GEMM plan: more than 8 rows");
+        require(scale_cols == 0 || scale_cols == 1 || scale_cols == ceil_div(K, 128), FP8LIN_ERR_ARGUMENT,
+                "GEMM plan: scale_cols must be 0 (BF16 weights), 1 or ceil(K/128)");
+        fp8lin::gemm_plan((int)scale_cols, (int)M, (int)N, (int)K, split != 0, plan[0], plan[1], plan[2], plan[3],
+                          plan[4]);
+    });
+}
+
 int fp8lin_linear_ws(const uint16_t* x, const uint8_t* codes, const float* scales, int64_t scale_cols,
                      uint16_t* y, int64_t M, int64_t N, int64_t K, int vector_gemv, void* workspace,
                      size_t workspace_bytes, fp8lin_stream_t stream) {

@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <atomic>
 
+#include "../../include/fp8lin.h"
 #include "gemm_fp8.hpp"
 #include "gemm_kernel.hpp"
 #include "internal.hpp"
@@ -237,9 +238,9 @@ float estimate(const gemm_fp8::Plan& p, int K, int G) {
 // the general template.  have: the bytes of workspace that K-split partials
 // may take; a plan that needs more is made without a split.  block: the
 // template's 256x256 tiles in the place of gemm_tile.hip's, where K allows and
-// they are one round on more than 0.6 of the CUs: 4096 x 2560 x 13440 316 us
-// against 345, 1036 x 8944 x 5248 129 against 141; median of 80 such shapes
-// 0.97, and 1.05 on fewer CUs, 1.03 over more rounds.  The persistent
+// they are one round on more than 0.6 of the CUs: 512 x 25088 x 5056 (SwiGLU)
+// 135 us against 147, 466 x 25656 x 4224 120 against 130; median of 80 such
+// shapes 0.97, and 1.05 on fewer CUs, 1.03 over more rounds.  The persistent
 // GEMM's unsplit sums do not depend on the row count or the tile height, and
 // the entry points that take no workspace (any false) keep them: there the
 // tiles only run the K that it does not.
@@ -290,6 +291,32 @@ size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu
     const Route r = route(nullptr, nullptr, S, ldy, M, N, K, swiglu, true, SIZE_MAX);
     const size_t gemm = gemm_split_bytes(S, ldy, M, N, K, swiglu);
     return r.tiles ? std::max(gemm, tile_plan_bytes(r.tile, M, N)) : gemm;
+}
+
+void gemm_plan(int S, int M, int N, int K, bool split, int& kind, int& bm, int& bn, int& splits, int& slots) {
+    bm = bn = splits = slots = 0;
+    kind = skinny(M, N, false) ? FP8LIN_GEMM_FEW_ROWS : FP8LIN_GEMM_ELEMENTS;
+    if (kind == FP8LIN_GEMM_FEW_ROWS) return;
+    if (S == 0) {
+        if (!tile_supported(nullptr, nullptr, false, 1, M, N, K)) return;
+        kind = FP8LIN_GEMM_TILES;
+        splits = 1;
+        return tile_shape(tile_plan(false, M, N, K, false), false, bm, bn, slots);
+    }
+    const Route r = route(nullptr, nullptr, S, N, M, N, K, false, split, split ? SIZE_MAX : 0);
+    if (mid_rows(nullptr, nullptr, S, M, N, K) || (r.gemm && r.plan.rtiles == 0 && halves(nullptr, nullptr, S, M, N, K))) {
+        kind = FP8LIN_GEMM_SMALL_M;
+    } else if (r.tiles) {
+        kind = r.block ? FP8LIN_GEMM_BLOCK : FP8LIN_GEMM_TILES;
+        splits = r.tile.splits;
+        tile_shape(r.tile, true, bm, bn, slots);
+    } else if (r.gemm) {
+        kind = FP8LIN_GEMM_PERSISTENT;
+        bm = r.plan.bm;
+        bn = gemm_fp8::BN;
+        slots = 1;
+        splits = r.plan.rtiles > 0 ? r.plan.splits : 1;
+    }
 }
 
 hipError_t launch_gemm_ws(const uint16_t* x, const void* w, const float* scales, int S, uint16_t* y, int64_t ldy,

@@ -155,6 +155,12 @@ TilePlan tile_plan(bool fp8, int M, int N, int K, bool may_split) {
 
 bool tile_is_block(const TilePlan& p) { return p.splits == 1 && kFp8[p.cfg].bm == 256 && kFp8[p.cfg].bn == 256; }
 
+void tile_shape(const TilePlan& p, bool fp8, int& bm, int& bn, int& slots) {
+    slots = tile_of(fp8, p.cfg).slots;
+    bm = tile_of(fp8, p.cfg).bm;
+    bn = tile_of(fp8, p.cfg).bn;
+}
+
 size_t tile_plan_bytes(const TilePlan& p, int M, int N) {
     return p.splits <= 1 ? 0 : (size_t)p.splits * M * (ceil_div(N, 8) * 8 + 8) * sizeof(float);
 }

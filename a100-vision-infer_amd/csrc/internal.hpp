@@ -76,6 +76,7 @@ struct TilePlan {
 bool tile_supported(const uint16_t* x, const void* w, bool fp8, int S, int64_t M, int64_t N, int64_t K);
 TilePlan tile_plan(bool fp8, int M, int N, int K, bool may_split);
 size_t tile_plan_bytes(const TilePlan& p, int M, int N);
+void tile_shape(const TilePlan& p, bool fp8, int& bm, int& bn, int& slots);
 bool tile_is_block(const TilePlan& p);  // FP8, whole 256x256 tiles
 hipError_t launch_tile(const TilePlan& p, bool fp8, const uint16_t* x, const void* w, const float* scales, int S,
                        const uint16_t* bias, uint16_t* y, int64_t ldy, int M, int N, int K, bool swiglu, void* ws,
@@ -97,6 +98,10 @@ hipError_t launch_gemm_bf16(const uint16_t* x, const uint16_t* w, const uint16_t
 // [M, N/2].
 size_t gemm_workspace_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
 size_t gemm_split_bytes(int S, int64_t ldy, int M, int N, int K, bool swiglu);
+// What a 16-byte aligned call of more than 8 rows runs (FP8LIN_GEMM_*), with its
+// tile and K ranges; S == 0: BF16 weights.
+void gemm_plan(int S, int M, int N, int K, bool split, int& kind, int& bm, int& bn, int& splits,
+               int& slots);
 // Whether the GEMM dispatch sends this FP8 call (9..32 rows) to the small-M
 // matrix-core kernel instead of a GEMM tile.
 bool gemm_mid_rows(const uint16_t* x, const void* w, int S, int64_t M, int64_t N, int64_t K);

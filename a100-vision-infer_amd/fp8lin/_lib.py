@@ -44,7 +44,7 @@ EXPORTED = [
     "fp8lin_linear_candidates_static",
     "fp8lin_linear_swiglu_workspace_bytes", "fp8lin_linear_swiglu_ws",
     "fp8lin_linear_workspace_bytes", "fp8lin_linear_ws",
-    "fp8lin_linear_scaled_workspace_bytes", "fp8lin_linear_swiglu_scaled_workspace_bytes",
+    "fp8lin_linear_scaled_workspace_bytes", "fp8lin_linear_swiglu_scaled_workspace_bytes", "fp8lin_gemm_plan",
     "fp8lin_decode_chain_workspace_bytes", "fp8lin_decode_chain",
 ]
 
@@ -112,6 +112,7 @@ def lib():
         "fp8lin_linear_ld": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i64, i32, vp]),
         "fp8lin_linear_workspace_bytes": (sz, [i64, i64, i64]),
         "fp8lin_linear_scaled_workspace_bytes": (sz, [i64, i64, i64, i64]),
+        "fp8lin_gemm_plan": (i32, [i64, i64, i64, i64, i32, ctypes.POINTER(i32)]),
         "fp8lin_decode_chain_workspace_bytes": (sz, [i32]),
         "fp8lin_decode_chain": (i32, [ctypes.POINTER(ChainLink), i32, vp, sz, vp]),
         "fp8lin_linear_ws": (i32, [vp, vp, vp, i64, vp, i64, i64, i64, i32, vp, sz, vp]),

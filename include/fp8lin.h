@@ -133,6 +133,23 @@ int fp8lin_linear_ws(const uint16_t* x, const uint8_t* codes, const float* scale
                      uint16_t* y, int64_t M, int64_t N, int64_t K, int vector_gemv, void* workspace,
                      size_t workspace_bytes, fp8lin_stream_t stream);
 
+/* What a call of more than 8 rows on 16-byte aligned operands runs: plan[0] is
+ * the kernel, plan[1] and plan[2] its tile's rows and columns, plan[3] the K
+ * ranges that its (last) tiles are cut into, plan[4] the workgroups per CU that
+ * it counts on (0 where it has no tiles).
+ * scale_cols 0: BF16 weights.  split: as the entry points with a workspace.
+ * Asks no device beyond its CU count (256 assumed without one); for tests and
+ * for reading timings. */
+enum {
+    FP8LIN_GEMM_FEW_ROWS = 0,   /* 256 weight rows or fewer */
+    FP8LIN_GEMM_SMALL_M = 1,    /* the small-M kernels, whole or in row halves */
+    FP8LIN_GEMM_PERSISTENT = 2,
+    FP8LIN_GEMM_TILES = 3,      /* one tile per workgroup */
+    FP8LIN_GEMM_BLOCK = 4,      /* the same by the 256x256 template */
+    FP8LIN_GEMM_ELEMENTS = 5    /* the template with element-wise loads */
+};
+int fp8lin_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t scale_cols, int split, int* plan);
+
 /* ---------------------------------------------------------------------------
  * Fused gate/up projection + SwiGLU: with G = fp8lin_linear(x, W) of shape
  * [M, N] (N even, rows [0, N/2) = gate, [N/2, N) = up, the row concatenation

@@ -367,6 +367,42 @@ def test_linear_workspace_bytes_by_scale_form(fp8lin, m, n, k):
     assert L.fp8lin_linear_swiglu_workspace_bytes(m, n, k) == need
 
 
+def _plan(fp8lin, m, n, k, cols, split):
+    out = (ctypes.c_int * 5)()
+    assert fp8lin.lib().fp8lin_gemm_plan(m, n, k, cols, int(split), out) == fp8lin.OK
+    return tuple(out)
+
+
+def test_gemm_plan(fp8lin):
+    """Which GEMM a call runs (256 CUs assumed): few weight rows and mid rows
+    first; K % 256 == 0 without a workspace stays on the persistent GEMM; a scale
+    form changes nothing else; the largest tiles stay at any K."""
+    few, small, persistent, tiles, block, elements = range(6)
+    assert _plan(fp8lin, 512, 48, 5120, 0, False)[0] == few
+    assert _plan(fp8lin, 512, 48, 5120, 40, True)[0] == few
+    assert _plan(fp8lin, 27, 17408, 5120, 40, True)[0] == small
+    assert _plan(fp8lin, 100, 5120, 8704, 68, False)[0] == small  # two row halves
+    assert _plan(fp8lin, 512, 17408, 5120, 40, False) == (persistent, 192, 256, 1, 1)
+    assert _plan(fp8lin, 4096, 17408, 5120, 40, False) == (persistent, 256, 256, 1, 1)
+    assert _plan(fp8lin, 4096, 17408, 5120, 40, True) == (persistent, 256, 256, 4, 1)
+    assert _plan(fp8lin, 300, 520, 641, 6, True)[0] == elements
+    assert _plan(fp8lin, 300, 520, 641, 0, False)[0] == elements
+    assert _plan(fp8lin, 512, 25088, 5056, 40, False)[:3] == (block, 256, 256)
+    for k in (7104, 9280, 13696, 24704, 34048 + 64):
+        kind, rows, cols = _plan(fp8lin, 4096, 8192, k, -(-k // 128), True)[:3]
+        assert kind == tiles and rows * cols >= 128 * 128
+    for m, n, k in ((9, 261, 1168), (93, 5120, 8704), (300, 8192, 3008), (129, 16400, 1168), (640, 17408, 5120)):
+        for split in (False, True):
+            a, b = _plan(fp8lin, m, n, k, 1, split), _plan(fp8lin, m, n, k, -(-k // 128), split)
+            assert a == b or b[0] == small
+            assert split or k % 256 or b[0] in (persistent, small)
+    out = (ctypes.c_int * 5)()
+    L = fp8lin.lib()
+    assert L.fp8lin_gemm_plan(8, 512, 512, 4, 0, out) == fp8lin.ERR_SHAPE
+    assert L.fp8lin_gemm_plan(64, 512, 512, 3, 0, out) == fp8lin.ERR_ARGUMENT
+    assert L.fp8lin_gemm_plan(64, 512, 512, 4, 0, None) == fp8lin.ERR_ARGUMENT
+
+
 def test_linear_ws_validation(fp8lin):
     """fp8lin_linear_ws checks its workspace before touching a device."""
     L = fp8lin.lib()

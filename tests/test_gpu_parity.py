@@ -236,8 +236,9 @@ def test_gemm_fp8(fp8lin, gpu, oracle, m, n, k):
 @pytest.mark.parametrize("n,k,swiglu", [(520, 512, False), (8200, 1024, False), (8200, 768, True),
                                         (17408, 5120, True)])
 def test_gemm_tile_heights_agree(fp8lin, gpu, oracle, n, k, swiglu):
-    """The FP8 GEMM runs 128-row tiles for M <= 128 and 256-row tiles above.
-    Unsplit, both give every output the same FP32 sum (same K order, same
+    """The FP8 GEMM runs 128-row tiles for M <= 128 and 192- or 256-row tiles
+    above (192 at these 129 rows; 256 in test_gpu_tile.py's own test).
+    Unsplit, all give every output the same FP32 sum (same K order, same
     accumulator position), so an M = 128 call equals rows 0..127 of an
     M = 129 call on the same rows bit for bit; the M = 128 call also holds
     the oracle bar (plain: a column sample, SwiGLU: all outputs of a row

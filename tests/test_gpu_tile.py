@@ -2,6 +2,8 @@
 edges of its tiles: every tile of its table, rows and columns one past a tile
 edge, column counts off the 8- and 16-column store groups, K ending inside a
 slice, a step and a ring."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -15,6 +17,16 @@ pytestmark = pytest.mark.gpu
 def sample(m):
     """All rows of a small call, else the first, the tile edges and the last."""
     return np.arange(m) if m <= 64 else np.unique(np.r_[0, 31, 32, 63, 64, 127, 128, m // 2, m - 2, m - 1].clip(0, m - 1))
+
+
+def plan(fp8lin, m, n, k, scale_cols, split):
+    """(kernel, tile rows, tile columns, K ranges, workgroups per CU) of a call."""
+    out = (ctypes.c_int * 5)()
+    fp8lin.check(fp8lin.lib().fp8lin_gemm_plan(m, n, k, scale_cols, int(split), out))
+    return tuple(out)
+
+
+FEW_ROWS, SMALL_M, PERSISTENT, TILES, BLOCK, ELEMENTS = range(6)
 
 
 # One row per tile (32x32, 64x32, 64x64, 128x64, 128x128 with K over two waves
@@ -123,12 +135,13 @@ def test_fp8_tile_long_k(fp8lin, gpu, oracle, m, n, k, rows_scaled):
         assert_parity(bits(y)[rows][:, cols], ref, f"long K {m}x{n}x{k} split={split}")
 
 
-@pytest.mark.parametrize("m,n,k", [(1036, 8944, 320), (512, 25090, 448), (466, 24578, 1216), (2048, 5382, 192)])
+@pytest.mark.parametrize("m,n,k", [(512, 25088, 320), (512, 25090, 448), (466, 24578, 1216), (705, 17410, 1344)])
 @pytest.mark.parametrize("rows_scaled", [False, True])
 def test_fp8_block_template(fp8lin, gpu, oracle, m, n, k, rows_scaled):
     """One round of 256x256 tiles on more than 0.6 of the CUs with K % 64 == 0:
     against the oracle, fused SwiGLU equal to the plain form's, a bias added to
     the rounded outputs, a row of NaN in its row."""
+    assert plan(fp8lin, m, n, k, 1 if rows_scaled else -(-k // 128), True)[0] == BLOCK
     rng = np.random.default_rng(m + n + k)
     codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
     scales = (rng.random(n if rows_scaled else (n, (k + 127) // 128)) * .01 + .001).astype(np.float32)
@@ -242,6 +255,137 @@ def test_dequant_branch_few_weight_rows(fp8lin, gpu, m, n, k, bias):
         assert_parity(bits(y), bits(ref), f"dequant {m}x{n}x{k}")
 
 
+# Every tile at a shape that runs it: rows one past a tile edge, ragged columns,
+# K that ends inside a step and spans two to three windows of scales.
+@pytest.mark.parametrize("tile,m,n,k", [
+    ((32, 32, 1), 9, 261, 1168), ((64, 32, 1), 33, 4100, 1168), ((64, 64, 1), 9, 8195, 1168), ((64, 128, 1), 9, 16400, 1168),
+    ((96, 64, 1), 65, 8195, 1168), ((96, 192, 1), 65, 16400, 1168), ((128, 64, 1), 97, 8195, 1168),
+    ((128, 128, 1), 97, 16400, 1168), ((128, 128, 2), 200, 16400, 1168), ((256, 256, 1), 769, 14340, 1168)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_every_fp8_tile(fp8lin, gpu, oracle, tile, m, n, k, rows_scaled):
+    assert plan(fp8lin, m, n, k, 1 if rows_scaled else -(-k // 128), False) == (TILES, *tile[:2], 1, tile[2])
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = np.exp2(-rng.integers(6, 12, n if rows_scaled else (n, -(-k // 128)))).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    rows, cols = sample(m), np.r_[0:65, n // 2:n // 2 + 65, n - 65:n]
+    y = fp8lin.fp8_linear(xd, cd, sd, split=False)
+    assert_parity(bits(y)[rows][:, cols], oracle.linear(x[rows], codes[cols], scales[cols]), f"tile {tile}")
+    if n % 2 == 0:
+        assert torch.equal(fp8lin.linear_swiglu(xd, cd, sd, split=False), fp8lin.fused_swiglu(y))
+
+
+@pytest.mark.parametrize("tile,m,n,k", [
+    ((32, 32, 1), 9, 261, 136), ((64, 32, 1), 33, 4100, 136), ((64, 64, 1), 9, 8195, 136), ((128, 64, 1), 65, 8195, 136),
+    ((128, 128, 1), 9, 16400, 136), ((128, 128, 2), 200, 16400, 136), ((192, 128, 1), 129, 16400, 136),
+    ((256, 160, 1), 385, 16400, 136), ((256, 256, 1), 1030, 12290, 136)])
+def test_every_bf16_tile(fp8lin, gpu, oracle, tile, m, n, k):
+    assert plan(fp8lin, m, n, k, 0, False) == (TILES, *tile[:2], 1, tile[2])
+    rng = np.random.default_rng(m + n + k)
+    x, w = rand_bf16(rng, (m, k)), rand_bf16(rng, (n, k), 0.05)
+    rows, cols = sample(m), np.r_[0:65, n // 2:n // 2 + 65, n - 65:n]
+    y = fp8lin.gemm_bf16(up(x, gpu), up(w, gpu))
+    assert_parity(bits(y)[rows][:, cols], oracle.linear_bf16w(x[rows], w[cols]), f"bf16 tile {tile}")
+
+
+# K ranges of every tile that takes them, with and without a bias.
+@pytest.mark.parametrize("tile,m,n,k", [
+    ((32, 32, 7), 9, 1030, 4112), ((64, 32, 7), 33, 1030, 4112), ((64, 64, 7), 9, 2052, 6160), ((64, 128, 7), 9, 4100, 6160),
+    ((96, 64, 7), 65, 1542, 6160), ((96, 192, 2), 65, 16400, 2192), ((128, 64, 7), 97, 2052, 6160),
+    ((128, 128, 7), 193, 2052, 6160), ((256, 256, 7), 193, 8195, 6160), ((96, 64, 3), 129, 2052, 4112)])
+def test_tile_k_ranges(fp8lin, gpu, oracle, tile, m, n, k):
+    """Against the oracle, the bias added to the rounded sums, and the same bits
+    again; fused SwiGLU equal to the plain form's where the pair halves are off
+    the 16-byte grid too."""
+    assert plan(fp8lin, m, n, k, -(-k // 128), True)[:4] == (TILES, *tile)
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = np.exp2(-rng.integers(6, 12, (n, -(-k // 128)))).astype(np.float32)
+    x, b = rand_bf16(rng, (m, k)), up(rand_bf16(rng, (n,)), gpu)
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    rows, cols = sample(m), np.r_[0:65, n // 2:n // 2 + 65, n - 65:n]
+    y = fp8lin.fp8_linear(xd, cd, sd)
+    assert_parity(bits(y)[rows][:, cols], oracle.linear(x[rows], codes[cols], scales[cols]), f"K ranges {tile}")
+    assert torch.equal(y, fp8lin.fp8_linear(xd, cd, sd))
+    eng = fp8lin.LinearEngine()
+    eng.add("p.weight", cd, sd)
+    eng.add("p.bias", b)
+    assert torch.equal(eng.linear(xd, "p"), fp8lin.add_bias(y.clone(), b))
+    if n % 2 == 0:
+        assert torch.equal(fp8lin.linear_swiglu(xd, cd, sd), fp8lin.fused_swiglu(y))
+
+
+@pytest.mark.parametrize("m,n,k,rows_scaled", [(65, 1542, 6160, False), (9, 1030, 4112, True), (65, 17408, 4096, False),
+                                               (97, 17408, 5120, False)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_workspace_of_any_size(fp8lin, gpu, oracle, m, n, k, rows_scaled, swiglu):
+    """From the size that a call is refused without (the persistent GEMM's
+    partials; none for K % 256 != 0) to more than the reported one, each meets
+    the bar and writes nothing behind the bytes it was given."""
+    L = fp8lin.lib()
+    cols = 1 if rows_scaled else -(-k // 128)
+    query = L.fp8lin_linear_swiglu_scaled_workspace_bytes if swiglu else L.fp8lin_linear_scaled_workspace_bytes
+    need = query(m, n, k, cols)
+    assert need > 0
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = np.exp2(-rng.integers(6, 12, n if rows_scaled else (n, cols))).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    out = n // 2 if swiglu else n
+    ref = fp8lin.fp8_linear(xd, cd, sd, split=False)
+    ref = bits(fp8lin.fused_swiglu(ref) if swiglu else ref)
+    kind, _, _, ranges, _ = plan(fp8lin, m, n, k, cols, True)
+    partials = ranges * m * (-(-n // 8) * 8 + 8) * 4 if kind == TILES and ranges > 1 else need
+    sizes = {need, need + 4096, max(partials, 16)} | ({partials - 16, 0} if k % 256 else set())
+    for size in sorted(sizes):
+        if k % 256 == 0 and size < need:
+            continue
+        ws = torch.full((size + 4096,), 0x5A, dtype=torch.uint8, device=gpu)
+        y = torch.empty((m, out), dtype=torch.bfloat16, device=gpu)
+        ptr = ws.data_ptr() if size else None
+        stream = torch.cuda.current_stream().cuda_stream
+        if swiglu:
+            rc = L.fp8lin_linear_swiglu_ws(xd.data_ptr(), cd.data_ptr(), sd.data_ptr(), cols, y.data_ptr(), m, n, k, ptr, size, stream)
+        else:
+            rc = L.fp8lin_linear_ws(xd.data_ptr(), cd.data_ptr(), sd.data_ptr(), cols, y.data_ptr(), m, n, k, 0, ptr, size, stream)
+        fp8lin.check(rc)
+        assert (ws[size:] == 0x5A).all(), f"{size} of {need} bytes"
+        assert_parity(bits(y), ref, f"workspace {size} of {need}", elementwise=False)
+
+
+# 256-row tiles of the persistent GEMM, unsplit (two tile rows at 200 to 512 rows
+# of a wide weight would be half padding at 192).
+@pytest.mark.parametrize("m,n,k", [(200, 33000, 512), (256, 34000, 512), (256, 33794, 1280), (512, 50000, 512), (2300, 7000, 768)])
+@pytest.mark.parametrize("rows_scaled", [False, True])
+def test_fp8_256_row_tiles(fp8lin, gpu, oracle, m, n, k, rows_scaled):
+    """Bit for bit the rows of a 128-row call, on 128-row tiles, which meets the
+    oracle; SwiGLU likewise; a row of NaN stays in its row."""
+    cols = 1 if rows_scaled else k // 128
+    assert plan(fp8lin, m, n, k, cols, False) == (PERSISTENT, 256, 256, 1, 1)
+    wide = n > 8192  # narrower weights run 65..128 rows as small-M halves
+    if wide:
+        assert plan(fp8lin, 128, n, k, cols, False) == (PERSISTENT, 128, 256, 1, 1)
+    rng = np.random.default_rng(m + n + k)
+    codes = rng.integers(0, 127, (n, k), dtype=np.uint8) | (rng.integers(0, 2, (n, k), dtype=np.uint8) << 7)
+    scales = (rng.random(n if rows_scaled else (n, cols)) * .01 + .001).astype(np.float32)
+    x = rand_bf16(rng, (m, k))
+    x[m // 2] = 0x7fc0  # NaN
+    xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
+    y = fp8lin.fp8_linear(xd, cd, sd, split=False)
+    assert torch.isnan(y[m // 2]).all()
+    if wide:
+        for i in (0, m - 128):
+            part = fp8lin.fp8_linear(xd[i:i + 128].contiguous(), cd, sd, split=False)
+            assert torch.equal(y[i:i + 128].nan_to_num(1e30), part.nan_to_num(1e30))
+    pair = fp8lin.linear_swiglu(xd, cd, sd, split=False)
+    assert torch.equal(pair.nan_to_num(1e30), fp8lin.fused_swiglu(y).nan_to_num(1e30))
+    rows = np.array([0, 127, m - 1])
+    cs = np.r_[0:64, n - 64:n]
+    assert_parity(bits(y)[rows][:, cs], oracle.linear(x[rows], codes[cs], scales[cs]), f"256-row tiles {m}x{n}x{k}")
+
+
 # 192-row tiles of the persistent GEMM (two or three rows of them in one round
 # where 256-row tiles fill half the chip to all of it): one row into a tile,
 # one short of it, whole, ragged columns, the fewest K steps that choose them.
@@ -257,6 +401,7 @@ def test_fp8_192_row_tiles(fp8lin, gpu, oracle, m, n, k, rows_scaled):
     scales = (rng.random(n if rows_scaled else (n, k // 128)) * .01 + .001).astype(np.float32)
     x = rand_bf16(rng, (m, k))
     x[m // 2] = 0x7fc0  # NaN
+    assert plan(fp8lin, m, n, k, 1 if rows_scaled else k // 128, False)[:2] == (PERSISTENT, 192)
     xd, cd, sd = up(x, gpu), up(codes, gpu), up(scales, gpu)
     y = fp8lin.fp8_linear(xd, cd, sd, split=False)
     assert torch.isnan(y[m // 2]).all()
