@@ -100,6 +100,7 @@ hipError_t run_fp8_mt(const uint16_t* x, const uint8_t* w, const float* scales, 
                       int M, int N, int K, const gemm_fp8::Plan& plan, int G, float* part, hipStream_t stream) {
     using namespace gemm_fp8;
     using Gm = Geo<MT>;
+    if (!Gm::SPLIT && plan.rtiles != 0) return hipErrorInvalidValue;
     auto kern = gemm_fp8_kernel<MT, SWIGLU>;
     static const hipError_t attr = gemm::allow_lds(reinterpret_cast<const void*>(kern), Gm::LDS_BYTES);
     if (attr != hipSuccess) return attr;
@@ -107,11 +108,14 @@ hipError_t run_fp8_mt(const uint16_t* x, const uint8_t* w, const float* scales, 
     hipLaunchKernelGGL(kern, dim3(grid), dim3(THREADS), Gm::LDS_BYTES, stream, x, w, scales, S, y, (int)ldy, M, N,
                        K, plan, part);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || plan.rtiles == 0) return e;
-    const int64_t threads = (int64_t)plan.rtiles * Gm::BM * (SWIGLU ? 32 : 64);
-    hipLaunchKernelGGL((tail_reduce_kernel<MT, SWIGLU>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                       stream, part, plan, M, N, y, ldy);
-    return hipGetLastError();
+    if constexpr (Gm::SPLIT) {
+        if (e != hipSuccess || plan.rtiles == 0) return e;
+        const int64_t threads = (int64_t)plan.rtiles * Gm::BM * (SWIGLU ? 32 : 64);
+        hipLaunchKernelGGL((tail_reduce_kernel<MT, SWIGLU>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
+                           stream, part, plan, M, N, y, ldy);
+        e = hipGetLastError();
+    }
+    return e;
 }
 
 template <bool SWIGLU>

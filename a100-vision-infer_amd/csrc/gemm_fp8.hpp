@@ -62,6 +62,7 @@ template <int MT>
 struct Geo {
     static_assert(MT == 4 || MT == 6 || MT == 8, "tile heights of 128, 192 or 256 rows");
     static constexpr int BM = 32 * MT;
+    static constexpr bool SPLIT = MT != 6;  // 192-row plans are unsplit
     static constexpr int A_STAGE = BM * 128;  // BM rows x 64 BF16
     static constexpr int A_BYTES = 3 * A_STAGE;
     static constexpr int LDS_BYTES = A_BYTES + 4 * B_WAVE;  // 160 KiB (MT 8), 136 KiB (MT 6) or 112 KiB (MT 4)
@@ -635,7 +636,7 @@ __global__ __launch_bounds__(256, 1) void gemm_fp8_kernel(const uint16_t* __rest
         // elements are read: with the accumulators live around the unit loop,
         // element reads straight from them made the register allocator move
         // every accumulator through scratch memory.
-        if (ep_slot >= 0) {
+        if (Gm::SPLIT && ep_slot >= 0) {
             // FP32 partial of a split tail tile: rows and columns in tile order.
             const rsrc_t rp = make_rsrc(part + (int64_t)ep_slot * Gm::SLOT_FLOATS, (uint32_t)(Gm::SLOT_FLOATS * 4));
             uint32_t voff[NT];

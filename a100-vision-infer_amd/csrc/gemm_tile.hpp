@@ -53,7 +53,7 @@ struct Cfg {
     static constexpr int ND = XD + WD;
     static constexpr int RING = ST * STAGE;
     static constexpr int SLICES = BK / 32;  // 32-K slices (two MFMAs deep) of a step
-    static_assert(BK == 32 || BK == 64 || BK == 128, "stages of whole 32-K slices");
+    static_assert(BK == 64 || BK == 128, "steps of half a 128-K block or a whole one");
     static_assert(ST >= (PIPE ? 3 : 2), "a stage in flight beside the ones read");
     static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0 && SLICES % WK == 0, "wave tile");
     static_assert(X_STAGE % (1024 * WAVES) == 0 && W_STAGE % (1024 * WAVES) == 0, "equal DMA shares");
@@ -165,8 +165,7 @@ template <int CH>
 __device__ __forceinline__ int swz(int r, int ch) {
     if constexpr (CH == 16) return ch ^ (r & 15);
     if constexpr (CH == 8) return ch ^ gemm_fp8::ga(r);
-    if constexpr (CH == 4) return ch ^ gemm_fp8::gb(r);
-    return ch ^ ((r >> 2) & 1);
+    return ch ^ gemm_fp8::gb(r);
 }
 
 // Column of fragment row i (0..31) in its 32-column block (see the header).
