@@ -137,6 +137,7 @@ __device__ __forceinline__ void store_staged(uint16_t* dst, int64_t ldy, const u
     static_assert(ITER % B == 0, "whole batches");
     const int lane = threadIdx.x & 63;
     asm volatile("" ::: "memory");  // the other lanes' rows, in the wave's own order
+#pragma unroll 1
     for (int p0 = 0; p0 < ITER; p0 += B) {
         Out v[B];
 #pragma unroll
