@@ -274,7 +274,7 @@ Route route(const uint16_t* x, const void* w, int S, int64_t ldy, int M, int N, 
         r.tile = tile_plan(true, M, N, K, any);
         if (tile_plan_bytes(r.tile, M, N) > have) r.tile = tile_plan(true, M, N, K, false);
         // against the plain form's plan for both epilogues: one route for both
-        r.tiles = (!r.gemm || r.tile.us < 0.95f * estimate(fitting(false), K, G));
+        r.tiles = (!r.gemm || r.tile.us < estimate(fitting(false), K, G));
     }
     if (r.tiles) r.gemm = false;
     const int64_t blocks = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
