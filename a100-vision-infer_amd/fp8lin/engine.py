@@ -243,14 +243,15 @@ class LinearEngine:
         wrote and read the [rows, N] product: 80 of 940 us of an MLP at 3913
         rows, a launch of 4 us at one row.  Other branches, and profiled calls
         (whose events time the projections alone), keep the two calls, and so
-        do 17..32 rows of a wide block-scaled weight off K 4097..5120, where
+        do 17..32 rows of a large block-scaled weight at K 2561..4096, where
         the small-M kernels' SwiGLU form takes up to 9% longer than the two
         (24 x 20480 x 3840 24.9 against 23.0 us, 27 x 28672 x 4096 32.7 against
-        30.4; 27 x 17408 x 5120 21.9 against 23.4)."""
+        30.4; 27 x 17408 x 5120 21.9 against 23.4).  Smaller ones are bound by
+        the host, which a second call costs 5 us."""
         if n.dim() == 2 and not self.profile_kernels and name not in self.mixed_projections:
             rec = self._record(name)
             rows = n.size(0)
-            slower = 16 < rows <= 32 and rec.N > 8192 and rec.scale_cols > 1 and not 4096 < rec.K <= 5120
+            slower = 16 < rows <= 32 and rec.scale_cols > 1 and 2560 < rec.K <= 4096 and rec.N * rec.K >= 1 << 26
             if not rec.bias and rec.N % 2 == 0 and not slower and lib().fp8lin_engine_linear_path(
                     ctypes.byref(self.options), ctypes.byref(rec), rows) in (PATH_FP8_GEMV, PATH_FP8_GEMM):
                 x = n.contiguous()
