@@ -369,7 +369,7 @@ int engine_branch(const fp8lin_linear_options& o, const fp8lin_weight& w, const 
     // bf16(decode(c) * s), the value every FP8 kernel here multiplies with, so
     // the FP8 kernels give it without a BF16 copy of the weight.  Slabs of
     // 2048 rows, each a dequantization and a GEMM of 8 column tiles, took 1640
-    // us for 640 x 17408 x 5120, where the FP8 GEMM takes 122.
+    // us for 640 x 17408 x 5120, where the FP8 GEMM takes 114.
     if (w.scales) {
         const size_t need = dequant_gemm_ws(w.N, w.K);
         require(ws != nullptr && ws_bytes >= need && aligned16(ws), FP8LIN_ERR_WORKSPACE,

@@ -65,7 +65,7 @@ struct Cfg {
     // FP8: the rows' scales, in two windows of SWB 128-K blocks beside the ring:
     // while the SPW steps of one run, SQ DMAs a wave fill the other.  Scales of
     // the whole K in LDS left no room for the large tiles at K above 8064
-    // (256x256): 1016 x 29884 x 11392 took 1074 us in smaller ones, 737 now.
+    // (256x256): 1016 x 29884 x 11392 took 1074 us in smaller ones, 634 in 256x256.
     // A DMA's 256 bytes hold 64 / SWB rows; the next ones start on another bank,
     // so that 32 rows at one block fall in distinct banks.
     static constexpr int SWB = BK == 128 ? 8 : 4, SPW = SWB * 128 / BK, SQ = FP8 ? BN * SWB / 64 / WAVES : 0;

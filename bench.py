@@ -39,7 +39,7 @@ PREFILL_TRAFFIC_BYTES = 1_119_044_894
 # the kernel changes.
 PREFILL_MFMA_BUSY = 0.723
 PREFILL_MFMA_BUSY_SOURCE = ("rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES GRBM_GUI_ACTIVE: 715.7e6 busy cycles "
-                            "/ 1024 SIMDs over GRBM_GUI_ACTIVE / 8 XCDs = 0.967e6 cycles (1.60 GHz)")
+                            "/ 1024 SIMDs over GRBM_GUI_ACTIVE / 8 XCDs = 0.967e6 cycles")
 SHAPES = [("gate_up", 17408, 5120), ("down", 5120, 8704), ("qkv_gate", 7168, 5120)]
 
 

@@ -119,8 +119,9 @@ int fp8lin_linear_ld(const uint16_t* x, const uint8_t* codes, const float* scale
  * K ranges and a second launch adds their FP32 sums in order and rounds
  * once.  Where smaller tiles, whole or in K ranges, are estimated faster
  * than that, they run instead.  Within the parity bar of fp8lin_linear (only
- * the FP32 summation order differs); up to 8 rows every call is
- * fp8lin_linear bit for bit.  The workspace is what
+ * the FP32 summation order differs, which M selects with the tile; so it does
+ * for BF16 weights, and without a workspace at K % 256 != 0); up to 8 rows
+ * every call is fp8lin_linear bit for bit.  The workspace is what
  * fp8lin_linear_workspace_bytes reports for block scales, and
  * fp8lin_linear_scaled_workspace_bytes for scale_cols of either form (0: none
  * needed), 16-byte aligned, any content.  Replaces the same `fp8_linear` as fp8lin_linear;
