@@ -31,19 +31,19 @@ constexpr Tile tile(int slots, float fixed, float tau, float tau1, float low) {
 }
 
 // BF16 weights, M x N x K in us (torch's mm, hipBLASLt, beside it): 1036 x 3456
-// x 1152 13.4 (24.5), 1036 x 4304 x 1152 18.0 (21.1), 1036 x 1152 x 4304 28
-// (31), 40 x 7168 x 5120 19.9 (22.3), 300 x 5120 x 5120 30.5 (35.8), 4096 x
-// 8192 x 8192 474 (355: the library's large tile is the better one).  The
-// 256x256-only kernel this replaced took 47, 46, 571 (K % 64 != 0), 159.
-// 192x128 and 256x160 stand where 128x128 would need another round of
-// workgroups or 256x256 leave CUs idle: 1036 x 4304 x 1152 18.0 (19.7 without
-// them), 1036 x 5120 x 5120 60 (76), 2048 x 4304 x 1152 28.5 (34.2), 2048 x
-// 5120 x 5120 103 (124), 4096 x 5120 x 5120 207 (236).
-// E4M3FN codes, M x N x K in us (before: the persistent GEMM or, at K % 256,
-// the general template): 93 x 17408 x 5120 40 (47), 93 x 5120 x 8704 25.7
-// (34.8), 200 x 7168 x 5120 33.6 (40.1), 512 x 2048 x 2048 11.9 (26.3), 320 x
-// 5120 x 3072 21.8 (33.7), 128 x 6000 x 1152 8.8 (20.2), 128 x 5000 x 4304
-// 21.6 (606, byte loads), row scales 27 x 8192 x 5120 14.3 (72.8).
+// x 1152 13.9 (24.5), 1036 x 4304 x 1152 18.1 (21.1), 1036 x 1152 x 4304 28
+// (31), 40 x 7168 x 5120 16.5 (22.3), 300 x 5120 x 5120 30.2 (35.8), 4096 x
+// 8192 x 8192 447 (355: the library's large tile is the better one).  The
+// 256x256-only kernel this replaced took 45, 45, 570 (K % 64 != 0), 156, 168
+// and 597.  192x128 and 256x160 stand where 128x128 would need another round
+// of workgroups or 256x256 leave CUs idle: 1036 x 4304 x 1152 18.0 (19.7
+// without them), 1036 x 5120 x 5120 60 (76), 2048 x 4304 x 1152 28.5 (34.2),
+// 2048 x 5120 x 5120 101 (124), 4096 x 5120 x 5120 203 (236).
+// E4M3FN codes, M x N x K in us (the persistent GEMM without these tiles or,
+// at K % 256, the general template): 93 x 17408 x 5120 36.8 (38.8), 93 x 5120 x
+// 8704 21.6 (28.5), 200 x 7168 x 5120 29.2 (37.1), 512 x 2048 x 2048 10.8
+// (26.1), 320 x 5120 x 3072 20.6 (33.7), 128 x 6000 x 1152 8.1 (18.8), 128 x
+// 5000 x 4304 18.4 (581, byte loads), row scales 27 x 8192 x 5120 14.1 (56.5).
 // What bounds them: at 128 rows or fewer the activations, which every
 // workgroup reads in full, share its 64 B/clk of DMA with the codes that come
 // from HBM (about 40 KB/us per CU against 29 for codes alone); above, LDS
